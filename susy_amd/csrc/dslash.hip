@@ -93,22 +93,24 @@ __device__ __forceinline__ float2 bload<float2>(Rsrc r, uint32_t voff, uint32_t 
 __device__ __forceinline__ int bload_i32(Rsrc r, uint32_t voff, uint32_t soff) {
   return (int)__builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, 0);
 }
-// cache policy of the output stores: non-temporal (2), so the written lines,
-// which this launch never reads again, do not displace the neighbour
-// gathers' source lines in L2 (FP32 CG iteration -0.8%, FP64 -1.8%)
-#ifndef DS_STORE_POLICY
-#define DS_STORE_POLICY 2
-#endif
-template <typename C> __device__ __forceinline__ void bstore(C v, Rsrc r, uint32_t voff, uint32_t soff);
+// cache policy of the output stores: k_dslash's are non-temporal (2), so the
+// written lines, which this launch never reads again, do not displace the
+// neighbour gathers' source lines in L2 (FP32 CG iteration -0.8%, FP64 -1.8%
+// at 12^3x24).  k_dslash_split's are ordinary ones (0): its fields fit L2,
+// and the next kernel finds them there (CG iteration, us, non-temporal ->
+// ordinary: U(2) 4^4 36.4 -> 31.1, U(3) 4^4 38.0 -> 34.7, U(4) 8^4 FP32 76.7
+// -> 75.0).
+#define DS_STORE_NT 2
+#define DS_STORE_L2 0
 // (callers keep the stored values live until the stores have read them:
 // hold() after the last store, see st_keep)
-template <>
-__device__ __forceinline__ void bstore<double2>(double2 v, Rsrc r, uint32_t voff, uint32_t soff) {
-  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(__attribute__((ext_vector_type(4))) unsigned, v), r, voff, soff, DS_STORE_POLICY);
+template <int POLICY>
+__device__ __forceinline__ void bstore(double2 v, Rsrc r, uint32_t voff, uint32_t soff) {
+  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(__attribute__((ext_vector_type(4))) unsigned, v), r, voff, soff, POLICY);
 }
-template <>
-__device__ __forceinline__ void bstore<float2>(float2 v, Rsrc r, uint32_t voff, uint32_t soff) {
-  __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(__attribute__((ext_vector_type(2))) unsigned, v), r, voff, soff, DS_STORE_POLICY);
+template <int POLICY>
+__device__ __forceinline__ void bstore(float2 v, Rsrc r, uint32_t voff, uint32_t soff) {
+  __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(__attribute__((ext_vector_type(2))) unsigned, v), r, voff, soff, POLICY);
 }
 
 // A matrix operand: field descriptor, lane byte offset of the site, uniform
@@ -153,6 +155,7 @@ __device__ __forceinline__ R bcsign(int t, int dt, int nt, R pbc) {
 // Pre-pass for the plaquette-determinant terms (doG): per site
 //   aux[0] = Tr eta,  aux[1+a] = Tr(U_a^-1 psi_a)
 // with eta, psi taken adjointed for D^dagger (utilities.c:793-799, 706-712).
+// One thread per site: for lattices whose sites fill the chip.
 template <typename R, bool DAG>
 __global__ void __launch_bounds__(256)
 k_dslash_prep(const typename CT<R>::t *__restrict__ src,
@@ -189,6 +192,46 @@ k_dslash_prep(const typename CT<R>::t *__restrict__ src,
   vm_drain();
 #pragma unroll
   for (int a = 0; a <= NUMLINK; a++) st_keep(aux + (size_t)a * V + s, t[a]);
+}
+
+// The same values with one thread per site and trace (blockIdx.y): six times
+// the waves hide the latency of a thread's loads.  The line lies where both
+// take the same time (us, pre-pass and D, k_dslash_prep | this, FP64): U(4)
+// 1296 sites 22.4 | 17.6, 8192 54.1 | 50.4, 65536 417.7 | 416.3; U(2) 8192
+// 16.8 | 15.6, 65536 95.4 | 96.9; at U(4) 131072 the pre-pass alone 60 | 67.
+#define PREP_TRACE_V 65536
+template <typename R, bool DAG>
+__global__ void __launch_bounds__(256)
+k_dslash_prep_trace(const typename CT<R>::t *__restrict__ src,
+                    const typename CT<R>::t *__restrict__ Uinv,
+                    typename CT<R>::t *__restrict__ aux, int V, const int *__restrict__ skip) {
+  typedef typename CT<R>::t C;
+  const int s = blockIdx.x * blockDim.x + threadIdx.x, k = blockIdx.y;
+  if (s >= V || (skip != nullptr && *skip)) return;
+  const C *psi = src + (size_t)k * NN * V + s;
+  C t = mkc<C>(0, 0);
+  if (k == 0) {
+#pragma unroll
+    for (int i = 0; i < NCOL; i++) {
+      const C v = psi[(i * NCOL + i) * V];
+      t.x += v.x;
+      t.y += DAG ? -v.y : v.y;
+    }
+  } else {
+    const C *ui = Uinv + (size_t)(k - 1) * NN * V + s;
+#pragma unroll
+    for (int i = 0; i < NCOL; i++)
+#pragma unroll
+      for (int j = 0; j < NCOL; j++) {
+        C u = ui[(i * NCOL + j) * V];
+        C p = DAG ? psi[(i * NCOL + j) * V] : psi[(j * NCOL + i) * V];
+        if (DAG) p.y = -p.y;
+        t.x += u.x * p.x - u.y * p.y;
+        t.y += u.x * p.y + u.y * p.x;
+      }
+  }
+  vm_drain();
+  st_keep(aux + (size_t)k * V + s, t);
 }
 
 template <typename R> struct DsSites;
@@ -458,7 +501,7 @@ k_dslash(const typename CT<R>::t *__restrict__ src, typename CT<R>::t *__restric
           v.y = fma(shift, q[i][k].y, v.y);
           dot += (double)q[i][k].x * (double)v.x + (double)q[i][k].y * (double)v.y;
         }
-        bstore<C>(v, rD, (uint32_t)s * cs, so);
+        bstore<DS_STORE_NT>(v, rD, (uint32_t)s * cs, so);
         out[i][k] = v;
       }
 #pragma unroll
@@ -500,6 +543,317 @@ k_dslash(const typename CT<R>::t *__restrict__ src, typename CT<R>::t *__restric
   }
 }
 
+#define DS_PARTS 5   // waves of k_dslash_split's block
+#if NCOL <= 4
+// The operator for lattices whose components and sites alone leave the chip
+// mostly idle: the ten products of an output matrix are shared by five waves
+// (two products each), which meet in LDS.  k_dslash makes them one after the
+// other, each behind its own loads, and that chain of memory latencies is
+// all its time on a small lattice.
+//
+// A block is 5 waves on one output component of 64 sites.  Wave w takes, for
+// the site, a = w; for link b, the w-th a != b or (w = 4) the StoL pair; for a
+// plaquette, one half of Dplus or (w >= 2) one PtoP pair.  The determinant
+// terms' sums over neighbours are shared the same way.
+//
+// What bounds it is still latency: gathered loads, then LDS and two barriers.
+// FP32 holds its partial matrices in two rounds of half the LDS and asks for
+// five waves per SIMD (U(4) D: four, what its registers allow without
+// scratch); FP64 asks for two, where fewer registers made it slower.
+// D with its pre-pass, us, FP64 | FP32, k_dslash -> this kernel:
+//   U(4) 4^3x8 23.7 -> 10.2 | 19.0 -> 9.4, 6^3x10 27.9 -> 23.3 | 24.9 -> 15.6
+//   U(3) 4^3x8 15.5 -> 8.0 | 13.9 -> 7.4, 6^3x10 19.3 -> 15.2 | 18.2 -> 11.3
+//   U(2) 4^4 10.2 -> 4.7 | 9.8 -> 4.7, 8^3x16 16.8 -> 14.7 | 16.7 -> 12.6
+// INL makes the pre-pass values in this kernel (ds_split_inline).
+template <typename R>
+constexpr int ds_split_waves(bool dag, bool inl) {
+  return sizeof(R) == 8 || inl ? 2 : NCOL == 4 && !dag ? 4 : 5;
+}
+template <typename R, bool DAG, int EPI, bool INL>
+__global__ void __launch_bounds__(64 * DS_PARTS)
+    __attribute__((amdgpu_waves_per_eu(ds_split_waves<R>(DAG, INL))))
+k_dslash_split(const typename CT<R>::t *__restrict__ src, typename CT<R>::t *__restrict__ dst,
+               const typename CT<R>::t *__restrict__ U,
+               const typename CT<R>::t *__restrict__ Uinv,
+               const typename CT<R>::t *__restrict__ pdet,
+               const typename CT<R>::t *__restrict__ aux, typename CT<R>::t *__restrict__ aux_out,
+               const int *__restrict__ nbr, const int *__restrict__ tco, int V, int nt, R pbc,
+               int doG, R G, DsOrder ord, const typename CT<R>::t *__restrict__ p0, R shift,
+               double *__restrict__ partial, const int *__restrict__ skip) {
+  typedef typename CT<R>::t C;
+  if (skip != nullptr && *skip) return;
+  // The partial matrices meet in LDS, ROUNDS times NR elements of them, and
+  // the determinant sums beside them
+  constexpr int ROUNDS = sizeof(R) == 8 ? 1 : 2, NR = (NN + ROUNDS - 1) / ROUNDS;
+  __shared__ C part[DS_PARTS][NR][64], dsum[DS_PARTS][64];
+  const int L = blockIdx.x, lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int q = L >> 3, comp = q % NTF, qq = q / NTF;
+  int s;
+  bool live;
+  if (ord.paired) {
+    const int par = qq & 1, pos = qq >> 1;
+    const int chunk = (L & 7) * ord.slab + (ord.paired == 2 ? (pos % ord.T) * ord.P + pos / ord.T : pos);
+    const int i = chunk * 64 + lane;
+    s = par ? ord.half + i : i;
+    live = i < (par ? V - ord.half : ord.half);
+  } else {
+    s = ((L & 7) * ord.slab + qq) * 64 + lane;
+    live = s < V;
+  }
+  if (!live) s = 0;   // computes site 0 again and stores nothing
+
+  const uint32_t cs = sizeof(C);
+  const uint32_t pl = (uint32_t)V * cs;     // one element plane
+  const uint32_t Mb = NN * pl;              // one matrix field
+  const Rsrc rS = make_rsrc(src, NTF * Mb), rU = make_rsrc(U, NUMLINK * Mb);
+  const Rsrc rN = make_rsrc(nbr, (uint32_t)NGATHER * V * 4u);
+  const Rsrc rA = make_rsrc(aux, 6 * pl), rP = make_rsrc(pdet, NUMLINK * NUMLINK * pl);
+  const Rsrc rI = make_rsrc(Uinv, NUMLINK * Mb);
+  auto nb = [&](int g) { return bload_i32(rN, (uint32_t)s * 4u, (uint32_t)g * V * 4u); };
+  auto S = [&](int k, int x) { return Opnd{rS, (uint32_t)x * cs, (uint32_t)k * Mb}; };
+  auto Ul = [&](int a, int x) { return Opnd{rU, (uint32_t)x * cs, (uint32_t)a * Mb}; };
+  auto num = [&](Rsrc r, int x, int k) { return bload<C>(r, (uint32_t)x * cs, k * pl); };
+  auto madd = [](C &sum, C a, C b, R f) {
+    sum.x += f * (a.x * b.x - a.y * b.y);
+    sum.y += f * (a.x * b.y + a.y * b.x);
+  };
+
+  // The pre-pass values Tr eta and Tr(U_c^-1 psi_c) at site x: read, or made
+  // here where the caller gives none, which costs the site component's waves
+  // ten more matrices but saves a launch
+  auto tr_eta = [&](int x) {
+    if (!INL) return num(rA, x, 0);
+    C v = mkc<C>(0, 0);
+#pragma unroll
+    for (int i = 0; i < NCOL; i++) {
+      const C e = num(rS, x, i * NCOL + i);
+      v.x += e.x;
+      v.y += DAG ? -e.y : e.y;
+    }
+    return v;
+  };
+  auto tr_psi = [&](int c, int x) {
+    if (!INL) return num(rA, x, 1 + c);
+    C v = mkc<C>(0, 0);
+#pragma unroll
+    for (int i = 0; i < NCOL; i++)
+#pragma unroll
+      for (int k = 0; k < NCOL; k++) {
+        C e = num(rS, x, (1 + c) * NN + (DAG ? i * NCOL + k : k * NCOL + i));
+        if (DAG) e.y = -e.y;
+        madd(v, num(rI, x, c * NN + i * NCOL + k), e, (R)1);
+      }
+    return v;
+  };
+
+  C acc[NCOL][NCOL], sum = mkc<C>(0, 0);
+#pragma unroll
+  for (int i = 0; i < NCOL; i++)
+#pragma unroll
+    for (int k = 0; k < NCOL; k++) acc[i][k] = mkc<C>(0, 0);
+  const int t = tco[s];
+  if (comp == 0) {
+    const int a = w, xm = nb(g_bwd(a));
+    const int xf = doG ? nb(g_fwd(a)) : s;
+    mmacc<R, DAG, true>(acc, (R)0.5, S(1 + a, s), Ul(a, s), pl);
+    mmacc<R, true, DAG>(acc, (R)-0.5 * bcsign<R>(t, -link_tau(a), nt, pbc), Ul(a, xm),
+                        S(1 + a, xm), pl);
+    if (doG) {
+      // sum_{c != a} plaqdet_ca(x) [T_a(x) + bc(a) T_c(x+a)]
+      const C ta = tr_psi(a, s);
+      const R sg = bcsign<R>(t, link_tau(a), nt, pbc);
+#pragma unroll
+      for (int n = 0; n < NUMLINK - 1; n++) {
+        const int c = n + (n >= a);
+        const C tc = tr_psi(c, xf);
+        madd(sum, num(rP, s, c * NUMLINK + a), mkc<C>(ta.x + sg * tc.x, ta.y + sg * tc.y), (R)1);
+      }
+    }
+  } else if (comp <= NUMLINK) {
+    const int b = comp - 1, xb = nb(g_fwd(b));
+    if (w < NUMLINK - 1) {
+      const int a = w + (w >= b), xm = nb(g_bwd(a)), pc = 6 + plaq_idx(a, b);
+      const R sg = a < b ? (R)1 : (R)-1;   // chi_ab = sg * stored chi_{min,max}
+      const R bc = bcsign<R>(t, -link_tau(a), nt, pbc);
+      mmacc<R, false, DAG>(acc, sg, Ul(a, xb), S(pc, s), pl);
+      mmacc<R, DAG, false>(acc, -sg * bc, S(pc, xm), Ul(a, xm), pl);
+      if (doG) {
+        // Tr eta(x) plaqdet_ab(x) + bc(-a) Tr eta(x-a) plaqdet_ba(x-a)
+        madd(sum, tr_eta(s), num(rP, s, a * NUMLINK + b), (R)1);
+        madd(sum, tr_eta(xm), num(rP, xm, b * NUMLINK + a), bc);
+      }
+    } else {
+      mmacc<R, DAG, true>(acc, (R)0.5 * bcsign<R>(t, link_tau(b), nt, pbc), S(0, xb), Ul(b, s),
+                          pl);
+      mmacc<R, true, DAG>(acc, (R)-0.5, Ul(b, s), S(0, s), pl);
+    }
+  } else {
+    const int p = comp - 1 - NUMLINK;
+    if (w < 2) {
+      // +-[bc(a) U_a(x) psi_b(x+a) + psi_a(x) U_b(x+a)], - with a, b exchanged
+      const int a = w ? c_pt.b[p] : c_pt.a[p], b = w ? c_pt.a[p] : c_pt.b[p];
+      const int xa = nb(g_fwd(a));
+      const R sg = w ? (R)-1 : (R)1;
+      mmacc<R, false, DAG>(acc, sg * bcsign<R>(t, link_tau(a), nt, pbc), Ul(a, s),
+                           S(1 + b, xa), pl);
+      mmacc<R, DAG, false>(acc, sg, S(1 + a, s), Ul(b, xa), pl);
+    } else {
+      // PtoP at double weight (see k_dslash)
+      const int n = w - 2, c = c_pt.pp_c[p][n], pc = 6 + c_pt.pp_de[p][n];
+      const int x1 = nb(c_pt.pp_g1[p][n]), x2 = nb(c_pt.pp_g2[p][n]), xmc = nb(g_bwd(c));
+      const R tr = (R)(2.0f * c_pt.pp_tr[p][n]);
+      mmacc<R, DAG, true>(acc, tr * bcsign<R>(t, c_pt.pp_dt3[p][n], nt, pbc), S(pc, x2),
+                          Ul(c, x1), pl);
+      mmacc<R, true, DAG>(acc, -tr * bcsign<R>(t, c_pt.pp_dt2[p][n], nt, pbc), Ul(c, xmc),
+                          S(pc, x1), pl);
+    }
+  }
+  // ---- the waves share the elements of the sum: of each round's, wave w
+  // takes w, w + 5, ...
+  constexpr int NE = (NR + DS_PARTS - 1) / DS_PARTS;
+  const bool det = doG && comp <= NUMLINK;
+  const bool pre = !DAG && EPI == 0 && aux_out != nullptr && comp <= NUMLINK;
+  C pq[ROUNDS][NE], u[ROUNDS][NE];
+#pragma unroll
+  for (int r = 0; r < ROUNDS; r++)
+#pragma unroll
+    for (int j = 0; j < NE; j++) {
+      const int e = min(r * NR + min(w + j * DS_PARTS, NR - 1), NN - 1);
+      pq[r][j] = u[r][j] = mkc<C>(0, 0);
+      if (EPI == 1)
+        pq[r][j] = bload<C>(make_rsrc(p0, NTF * Mb), (uint32_t)s * cs,
+                            comp * Mb + (DAG ? (e % NCOL) * NCOL + e / NCOL : e) * pl);
+      // element e of U^-1 as the accumulator holds it
+      if ((det || pre) && comp > 0)
+        u[r][j] = bload<C>(rI, (uint32_t)s * cs, (comp - 1) * Mb + e * pl);
+    }
+  dsum[w][lane] = sum;
+  double dot = 0;
+  C tr = mkc<C>(0, 0);
+  const Rsrc rD = make_rsrc(dst, NTF * Mb);
+#pragma unroll
+  for (int r = 0; r < ROUNDS; r++) {
+    if (r) __syncthreads();   // the last round's elements have been read
+#pragma unroll
+    for (int e = 0; e < NR; e++)
+      if (r * NR + e < NN) part[w][e][lane] = acc[(r * NR + e) / NCOL][(r * NR + e) % NCOL];
+    __syncthreads();
+    if (r == 0 && det) {
+      sum = mkc<C>(0, 0);
+#pragma unroll
+      for (int i = 0; i < DS_PARTS; i++) {
+        const C v = dsum[i][lane];
+        sum.x += v.x;
+        sum.y += v.y;
+      }
+      const R f = (R)(comp == 0 ? 0.5 * C2 : -0.5 * C2) * G;
+      sum.x *= f;
+      sum.y *= f;
+    }
+#pragma unroll
+    for (int j = 0; j < NE; j++) {
+      const int er = w + j * DS_PARTS, e = r * NR + er;
+      if (er >= NR || e >= NN) continue;
+      C v = mkc<C>(0, 0);
+#pragma unroll
+      for (int i = 0; i < DS_PARTS; i++) {
+        const C x = part[i][er][lane];
+        v.x += x.x;
+        v.y += x.y;
+      }
+      const bool diag = e / NCOL == e % NCOL;
+      const C ue = u[r][j];
+      if (det) {
+        if (comp > 0) {
+          v.x += sum.x * ue.x - sum.y * ue.y;
+          v.y += sum.x * ue.y + sum.y * ue.x;
+        } else if (diag) {
+          v.x += sum.x;
+          v.y += sum.y;
+        }
+      }
+      if (pre) {
+        // Tr(out_0)^*, or Tr(U^-1 out^dagger)
+        if (comp > 0) {
+          tr.x += ue.x * v.x + ue.y * v.y;
+          tr.y += ue.y * v.x - ue.x * v.y;
+        } else if (diag) {
+          tr.x += v.x;
+          tr.y -= v.y;
+        }
+      }
+      // D^dagger: element (i,k) of the accumulator is minus the conjugate of
+      // element (k,i) of the result
+      const int d = DAG ? (e % NCOL) * NCOL + e / NCOL : e;
+      if (DAG) v.x = -v.x;
+      if (EPI == 1) {
+        const C x = pq[r][j];
+        v.x = fma(shift, x.x, v.x);
+        v.y = fma(shift, x.y, v.y);
+        dot += (double)x.x * (double)v.x + (double)x.y * (double)v.y;
+      }
+      if (live) {
+        bstore<DS_STORE_L2>(v, rD, (uint32_t)s * cs, comp * Mb + d * pl);
+        hold(v);
+      }
+    }
+  }
+  if (pre) {
+    __syncthreads();   // the determinant sums have been read
+    dsum[w][lane] = tr;
+    __syncthreads();
+    if (w == 0 && live) {
+      tr = mkc<C>(0, 0);
+#pragma unroll
+      for (int i = 0; i < DS_PARTS; i++) {
+        const C v = dsum[i][lane];
+        tr.x += v.x;
+        tr.y += v.y;
+      }
+      st_keep(aux_out + (size_t)comp * V + s, tr);
+    }
+  }
+  if (EPI == 1) {
+    if (!live) dot = 0;
+    for (int off = 32; off > 0; off >>= 1) dot += __shfl_xor(dot, off, 64);
+    __shared__ double red[DS_PARTS];
+    if (lane == 0) red[w] = dot;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      double tsum = 0;
+      for (int i = 0; i < DS_PARTS; i++) tsum += red[i];
+      partial[L] = tsum;
+      hold(tsum);
+    }
+  }
+}
+
+// The lattices k_dslash_split is for.  It reads each operand about half as
+// often beyond L2 as k_dslash, but keeps fewer loads in flight per wave, so
+// k_dslash wins where a launch fills the chip.  Both sides, us of a CG
+// iteration, which leaves less of the operands in the caches than an operator
+// that is repeated alone, k_dslash | k_dslash_split:
+//   U(4) FP64  1296: 87.0 | 62.2    2160: 93.0 | 78.5    4096: 105.9 | 103.0
+//              8192: 168.9 | 183.6  (4096 sites alone: D 27.3 | 29.6)
+//        FP32  2160: 78.4 | 61.5    4096: 83.1 | 76.5    8192: 117.2 | 122.9
+//   U(3) FP64  1296: 61.5 | 48.0    2160: 64.2 | 57.5    4096: 68.2 | 71.9
+//        FP32  8192: 80.2 | 75.5   20736: 162.2 | 149.8 65536: 420.3 | 423.2
+//   U(2) FP64  8192: 62.8 | 61.9   20736: 136.8 | 116.6 65536: 320.7 | 328.2
+//        FP32  8192: 56.3 | 52.8   20736: 96.7 | 86.9   65536: 208.5 | 210.2
+template <typename R>
+static bool ds_split(int V) {
+  const bool dbl = sizeof(R) == sizeof(double);
+  return V <= (NCOL == 2 || (NCOL == 3 && !dbl) ? 32768 : dbl ? 3072 : 6144);
+}
+
+// Where it also makes the pre-pass values itself: the launch of k_dslash_prep
+// is 1.6 us of 6.3 on U(2) 4^4 and still wins a little at 6^4 (7.7 -> 7.5);
+// with the larger matrices the ten more products cost more than it (U(3) 4^4
+// 7.9 -> 10.0, U(4) 4^3x8 10.2 -> 12.3).
+static constexpr bool ds_split_inline(int V) { return NCOL == 2 && V <= 1296; }
+#endif  // NCOL <= 4
+
 template <typename R>
 static int dslash_launch(susy_ctx *c, const typename CT<R>::t *src,
                          typename CT<R>::t *dst, int sign, const typename CT<R>::t *p0,
@@ -518,21 +872,32 @@ static int dslash_launch(susy_ctx *c, const typename CT<R>::t *src,
     return SUSY_E_ARG;
   }
   if (sign != 1 || p0 != nullptr || !c->doG) aux_out = nullptr;
-  if (c->doG && prep) {
-    int nb = (V + 255) / 256;
-    if (sign == 1)
-      hipLaunchKernelGGL((k_dslash_prep<R, false>), dim3(nb), dim3(256), 0, c->s, src, Uinv, aux, V,
-                         skip);
-    else
-      hipLaunchKernelGGL((k_dslash_prep<R, true>), dim3(nb), dim3(256), 0, c->s, src, Uinv, aux, V,
-                         skip);
+#if NCOL <= 4
+  const bool split = ds_split<R>(V), inl = split && c->doG && prep && ds_split_inline(V);
+#else
+  const bool split = false, inl = false;
+#endif
+  if (c->doG && prep && !inl) {
+    const int nbp = (V + 255) / 256;
+#define PREP_GO(KERNEL, GRID)                                                          \
+  do {                                                                                 \
+    if (sign == 1)                                                                     \
+      hipLaunchKernelGGL((KERNEL<R, false>), GRID, dim3(256), 0, c->s, src, Uinv, aux, \
+                         V, skip);                                                     \
+    else                                                                               \
+      hipLaunchKernelGGL((KERNEL<R, true>), GRID, dim3(256), 0, c->s, src, Uinv, aux,  \
+                         V, skip);                                                     \
+  } while (0)
+    if (V <= PREP_TRACE_V) PREP_GO(k_dslash_prep_trace, dim3(nbp, 1 + NUMLINK));
+    else PREP_GO(k_dslash_prep, dim3(nbp));
+#undef PREP_GO
     HIPCHK(hipGetLastError());
   }
   DsOrder ord;
-  constexpr int threads = DsSites<R>::n * DS_SPLIT * DsSites<R>::cpb;
+  const int threads = split ? 64 * DS_PARTS : DsSites<R>::n * DS_SPLIT * DsSites<R>::cpb;
   const int nb = ds_grid(V, c->p.nx * c->p.ny * c->p.nz,
                          sizeof(R) == sizeof(float) ? c->site_order32 : c->site_order,
-                         DsSites<R>::n, &ord, DsSites<R>::cpb);
+                         split ? 64 : DsSites<R>::n, &ord, split ? 1 : DsSites<R>::cpb);
   if (nblocks) *nblocks = nb;
   R pbc = (R)c->p.PBC, G = (R)c->p.G;
 #define DS_ARGS src, dst, U, Uinv, pdet, aux, aux_out, c->d_nbr, c->d_t, V, c->p.nt, pbc, \
@@ -547,17 +912,30 @@ static int dslash_launch(susy_ctx *c, const typename CT<R>::t *src,
     HIPCHK(hipEventRecord(e0, c->s));
   }
   const unsigned lds = sizeof(R) == sizeof(double) ? DS_OCC_LDS64 : DS_OCC_LDS32;
+#if NCOL <= 4
+#define DS_GO(DAG, EPI)                                                                       \
+  do {                                                                                        \
+    if (inl)                                                                                  \
+      hipLaunchKernelGGL((k_dslash_split<R, DAG, EPI, NCOL == 2>), dim3(nb), dim3(threads),   \
+                         0, c->s, DS_ARGS);                                                   \
+    else if (split)                                                                           \
+      hipLaunchKernelGGL((k_dslash_split<R, DAG, EPI, false>), dim3(nb), dim3(threads), 0,    \
+                         c->s, DS_ARGS);                                                      \
+    else                                                                                      \
+      hipLaunchKernelGGL((k_dslash<R, DAG, EPI>), dim3(nb), dim3(threads), lds, c->s, DS_ARGS); \
+  } while (0)
+#else
+#define DS_GO(DAG, EPI) \
+  hipLaunchKernelGGL((k_dslash<R, DAG, EPI>), dim3(nb), dim3(threads), lds, c->s, DS_ARGS)
+#endif
   if (p0 == nullptr) {
-    if (sign == 1)
-      hipLaunchKernelGGL((k_dslash<R, false, 0>), dim3(nb), dim3(threads), lds, c->s, DS_ARGS);
-    else
-      hipLaunchKernelGGL((k_dslash<R, true, 0>), dim3(nb), dim3(threads), lds, c->s, DS_ARGS);
+    if (sign == 1) DS_GO(false, 0);
+    else DS_GO(true, 0);
   } else {
-    if (sign == 1)
-      hipLaunchKernelGGL((k_dslash<R, false, 1>), dim3(nb), dim3(threads), lds, c->s, DS_ARGS);
-    else
-      hipLaunchKernelGGL((k_dslash<R, true, 1>), dim3(nb), dim3(threads), lds, c->s, DS_ARGS);
+    if (sign == 1) DS_GO(false, 1);
+    else DS_GO(true, 1);
   }
+#undef DS_GO
 #undef DS_ARGS
   HIPCHK(hipGetLastError());
   if (e0) {
