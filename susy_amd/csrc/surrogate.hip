@@ -212,17 +212,15 @@ __device__ __forceinline__ int opp_tap(int t) { return t == 0 ? 0 : ((t & 1) ? t
 
 __device__ __forceinline__ void load_op(Mat m, const double2 *__restrict__ U, int a, int site,
                                         int dg, int V) {
+  // (the factor and its conjugation may differ between lanes)
   const double2 *p = U + (size_t)a * NN * V + site;
+  const int si = dg ? V : NCOL * V, sj = dg ? NCOL * V : V;
 #pragma unroll
   for (int i = 0; i < NCOL; i++)
 #pragma unroll
     for (int j = 0; j < NCOL; j++) {
-      if (dg) {
-        double2 v = p[(j * NCOL + i) * V];
-        m[i][j] = make_double2(v.x, -v.y);
-      } else {
-        m[i][j] = p[(i * NCOL + j) * V];
-      }
+      const double2 v = p[i * si + j * sj];
+      m[i][j] = make_double2(v.x, dg ? -v.y : v.y);
     }
 }
 __device__ __forceinline__ void mmul_into(Mat acc, const Mat f) {   // acc = acc f
@@ -234,141 +232,210 @@ __device__ __forceinline__ void mmul_into(Mat acc, const Mat f) {   // acc = acc
 #pragma unroll
     for (int j = 0; j < NCOL; j++) acc[i][j] = t[i][j];
 }
-__device__ __forceinline__ double2 mtrace(const Mat m) {
+// Block -> (chunk of sites, part of the chunk's work): all parts of a chunk on
+// one XCD after each other, and neighbouring chunks on the same XCD, so the
+// links that loops share are found in its L2 (workgroups go round-robin over
+// the 8 XCDs).  Grid sg_grid; false: no such chunk.
+static int sg_grid(int chunks, int parts) { return (chunks + 7) / 8 * 8 * parts; }
+__device__ __forceinline__ bool sg_block(int chunks, int parts, int *chunk, int *part) {
+  const int L = blockIdx.x, q = L >> 3;
+  *part = q % parts;
+  *chunk = (L & 7) * ((chunks + 7) / 8) + q / parts;
+  return *chunk < chunks;
+}
+
+// Tr(a b)
+__device__ __forceinline__ double2 mtrace_mul(const Mat a, const Mat b) {
   double2 t = make_double2(0, 0);
 #pragma unroll
-  for (int i = 0; i < NCOL; i++) {
-    t.x += m[i][i].x;
-    t.y += m[i][i].y;
-  }
+  for (int i = 0; i < NCOL; i++)
+#pragma unroll
+    for (int j = 0; j < NCOL; j++) {
+      t.x += a[i][j].x * b[j][i].x - a[i][j].y * b[j][i].y;
+      t.y += a[i][j].x * b[j][i].y + a[i][j].y * b[j][i].x;
+    }
   return t;
 }
 
 // ---------------------------------------------------------------------
-// features phi[k * V + y]
-__global__ void __launch_bounds__(SGB)
+// features phi[k * V + y], one thread per site and loop (blockIdx.y < 30) or
+// link norm.  What bounds it on a small lattice is a loop's chain of loads
+// and products, on a large one what the XCDs' L2 miss; one thread per site
+// walked all 30 loops (us: U(4) 4^3x8 306 -> 12, 16^4 508 -> 221, U(2) 16^4
+// 114 -> 36).
+#define SGF_B 64
+__global__ void __launch_bounds__(SGF_B)
 k_sg_features(const double2 *__restrict__ U, const int *__restrict__ base,
               float *__restrict__ phi, int V) {
-  const int y = blockIdx.x * SGB + threadIdx.x;
+  int chunk, k;
+  if (!sg_block((V + SGF_B - 1) / SGF_B, SG_NLOOP + NUMLINK, &chunk, &k)) return;
+  const int y = chunk * SGF_B + threadIdx.x;
   if (y >= V) return;
-#pragma unroll 1
-  for (int k = 0; k < SG_NLOOP; k++) {
-    Mat acc, f;
-    load_op(acc, U, c_sg.fdir[k][0], base[c_sg.foff[k][0] * V + y], c_sg.fdag[k][0], V);
-#pragma unroll 1
-    for (int m = 1; m < c_sg.nfac[k]; m++) {
-      load_op(f, U, c_sg.fdir[k][m], base[c_sg.foff[k][m] * V + y], c_sg.fdag[k][m], V);
-      mmul_into(acc, f);
-    }
-    double2 tr = mtrace(acc);
-    ST(phi[(size_t)(2 * k) * V + y], (float)(tr.x / NCOL));
-    ST(phi[(size_t)(2 * k + 1) * V + y], (float)(tr.y / NCOL));
-  }
-#pragma unroll 1
-  for (int a = 0; a < NUMLINK; a++) {
+  if (k >= SG_NLOOP) {
+    const int a = k - SG_NLOOP;
     const double2 *p = U + (size_t)a * NN * V + y;
     double s = 0;
+#pragma unroll
     for (int e = 0; e < NN; e++) {
       double2 v = p[(size_t)e * V];
       s += v.x * v.x + v.y * v.y;
     }
     ST(phi[(size_t)(60 + a) * V + y], (float)(s / NCOL - 1.0));
+    return;
   }
+  const int n = c_sg.nfac[k];
+  Mat acc, f;
+  load_op(acc, U, c_sg.fdir[k][0], base[c_sg.foff[k][0] * V + y], c_sg.fdag[k][0], V);
+#pragma unroll 1
+  for (int m = 1; m < n - 1; m++) {
+    load_op(f, U, c_sg.fdir[k][m], base[c_sg.foff[k][m] * V + y], c_sg.fdag[k][m], V);
+    mmul_into(acc, f);
+  }
+  load_op(f, U, c_sg.fdir[k][n - 1], base[c_sg.foff[k][n - 1] * V + y], c_sg.fdag[k][n - 1], V);
+  const double2 tr = mtrace_mul(acc, f);
+  ST(phi[(size_t)(2 * k) * V + y], (float)(tr.x / NCOL));
+  ST(phi[(size_t)(2 * k + 1) * V + y], (float)(tr.y / NCOL));
 }
 
-// v = d/dt phi(U + t R)
-__global__ void __launch_bounds__(SGB)
+// v = d/dt phi(U + t R), split like the features
+__global__ void __launch_bounds__(SGF_B)
 k_sg_jvp(const double2 *__restrict__ U, const double2 *__restrict__ R,
          const int *__restrict__ base, float *__restrict__ v, int V) {
-  const int y = blockIdx.x * SGB + threadIdx.x;
+  int chunk, k;
+  if (!sg_block((V + SGF_B - 1) / SGF_B, SG_NLOOP + NUMLINK, &chunk, &k)) return;
+  const int y = chunk * SGF_B + threadIdx.x;
   if (y >= V) return;
-#pragma unroll 1
-  for (int k = 0; k < SG_NLOOP; k++) {
-    const int n = c_sg.nfac[k];
-    double2 tot = make_double2(0, 0);
-#pragma unroll 1
-    for (int r = 0; r < n; r++) {
-      Mat acc, f;
-      load_op(acc, r == 0 ? R : U, c_sg.fdir[k][0], base[c_sg.foff[k][0] * V + y],
-              c_sg.fdag[k][0], V);
-#pragma unroll 1
-      for (int m = 1; m < n; m++) {
-        load_op(f, r == m ? R : U, c_sg.fdir[k][m], base[c_sg.foff[k][m] * V + y],
-                c_sg.fdag[k][m], V);
-        mmul_into(acc, f);
-      }
-      double2 tr = mtrace(acc);
-      tot.x += tr.x;
-      tot.y += tr.y;
-    }
-    ST(v[(size_t)(2 * k) * V + y], (float)(tot.x / NCOL));
-    ST(v[(size_t)(2 * k + 1) * V + y], (float)(tot.y / NCOL));
-  }
-#pragma unroll 1
-  for (int a = 0; a < NUMLINK; a++) {
+  if (k >= SG_NLOOP) {
+    const int a = k - SG_NLOOP;
     const double2 *p = U + (size_t)a * NN * V + y, *q = R + (size_t)a * NN * V + y;
     double s = 0;
+#pragma unroll
     for (int e = 0; e < NN; e++) {
       double2 u = p[(size_t)e * V], w = q[(size_t)e * V];
       s += u.x * w.x + u.y * w.y;
     }
     ST(v[(size_t)(60 + a) * V + y], (float)(2.0 * s / NCOL));
+    return;
   }
+  const int n = c_sg.nfac[k];
+  double2 tot = make_double2(0, 0);
+#pragma unroll 1
+  for (int r = 0; r < n; r++) {
+    Mat acc, f;
+    load_op(acc, r == 0 ? R : U, c_sg.fdir[k][0], base[c_sg.foff[k][0] * V + y],
+            c_sg.fdag[k][0], V);
+#pragma unroll 1
+    for (int m = 1; m < n - 1; m++) {
+      load_op(f, r == m ? R : U, c_sg.fdir[k][m], base[c_sg.foff[k][m] * V + y],
+              c_sg.fdag[k][m], V);
+      mmul_into(acc, f);
+    }
+    load_op(f, r == n - 1 ? R : U, c_sg.fdir[k][n - 1], base[c_sg.foff[k][n - 1] * V + y],
+            c_sg.fdag[k][n - 1], V);
+    const double2 tr = mtrace_mul(acc, f);
+    tot.x += tr.x;
+    tot.y += tr.y;
+  }
+  ST(v[(size_t)(2 * k) * V + y], (float)(tot.x / NCOL));
+  ST(v[(size_t)(2 * k + 1) * V + y], (float)(tot.y / NCOL));
 }
 
 // out[o](s) = sum_t sum_i W[t][o][i] in[i](s + d_t)       (ADJ = false)
 // out[i](s) = sum_t sum_o W[t][o][i] in[o](s - d_t)       (ADJ = true)
 // W in bfloat16, row-major [t][o][i] with o < CO, i < CI.
-template <int CI, int CO, bool ADJ>
-__device__ __forceinline__ void conv_site(const unsigned short *__restrict__ W,
-                                          const float *__restrict__ in,
-                                          const int *__restrict__ nbr, int s, int V,
-                                          float *out) {
-  constexpr int NOUT = ADJ ? CI : CO, NIN = ADJ ? CO : CI;
+//
+// A contraction over taps and channels, made for 16 sites a block with
+// v_mfma_f32_16x16x4_f32 (weights widened to FP32, inputs and sums FP32 as
+// before): rows are outputs, columns sites.  A lane's four inputs of the
+// channel sum belong to its quarter of the channels, so any order of them
+// serves both operands.  The block's waves are the 16-output tiles times TG
+// groups of taps, whose partial tiles meet in LDS.  What bounds it is the
+// latency of one round of gathered loads; one thread per site had 11440
+// dependent multiply-adds in conv1.  us at 4^3x8 | 16^4: conv1 131 -> 4.9 |
+// 169 -> 60, conv2 38 -> 3.5 | 50 -> 14, back1 32 -> 3.5 | 41 -> 12, back0
+// 163 -> 4.3 | 200 -> 48.
+typedef __attribute__((ext_vector_type(4))) float f32x4;
+#define CV_SITES 16
+template <int CI, int CO, bool ADJ, int TG>
+struct Conv {
+  static constexpr int nout = ADJ ? CI : CO, nin = ADJ ? CO : CI;
+  static constexpr int tiles = (nout + 15) / 16, threads = 64 * tiles * TG;
+  float red[TG][tiles * 16][CV_SITES];
+
+  // all threads of the block; at() may be read afterwards
+  __device__ __forceinline__ void run(const unsigned short *__restrict__ W,
+                                      const float *__restrict__ in,
+                                      const int *__restrict__ nbr, int s0, int V) {
+    constexpr int kq = (nin + 3) / 4;   // channels of a quarter of the lanes
+    const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int tile = w % tiles, tg = w / tiles, col = threadIdx.x & 15, g = (threadIdx.x & 63) >> 4;
+    const int s = min(s0 + col, V - 1), row = tile * 16 + col;
+    f32x4 acc[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
 #pragma unroll
-  for (int q = 0; q < NOUT; q++) out[q] = 0.f;
-#pragma unroll 1
-  for (int t = 0; t < SG_NT; t++) {
-    const int x = tap_site(nbr, ADJ ? opp_tap(t) : t, s, V);
-    const unsigned short *Wt = W + t * CO * CI;
-#pragma unroll 1
-    for (int p = 0; p < NIN; p++) {
-      const float xin = in[(size_t)p * V + x];
+    for (int n = 0; n < (SG_NT + TG - 1) / TG; n++) {
+      const int t = tg + n * TG;
+      if (t >= SG_NT) break;
+      const int x = tap_site(nbr, ADJ ? opp_tap(t) : t, s, V);
+      const unsigned short *Wt = W + t * CO * CI;
+      float wv[kq], xv[kq];
 #pragma unroll
-      for (int q = 0; q < NOUT; q++) {
-        const float w = ADJ ? bf2f(Wt[p * CI + q]) : bf2f(Wt[q * CI + p]);
-        out[q] = fmaf(w, xin, out[q]);
+      for (int m = 0; m < kq; m++) {
+        const int k = min(g * kq + m, nin - 1), r = min(row, nout - 1);
+        wv[m] = bf2f(ADJ ? Wt[k * CI + r] : Wt[r * CI + k]);
+        xv[m] = in[(size_t)k * V + x];
+      }
+      __builtin_amdgcn_sched_barrier(0);   // (one round of loads, then the products)
+#pragma unroll
+      for (int m = 0; m < kq; m++) {
+        const bool live = g * kq + m < nin;
+        acc[m & 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(live ? wv[m] : 0.f,
+                                                          live ? xv[m] : 0.f, acc[m & 1], 0, 0, 0);
       }
     }
+#pragma unroll
+    for (int r = 0; r < 4; r++) red[tg][tile * 16 + 4 * g + r][col] = acc[0][r] + acc[1][r];
+    __syncthreads();
   }
-}
+  // output e = q * CV_SITES + site
+  __device__ __forceinline__ float at(int e) const {
+    float z = 0;
+#pragma unroll
+    for (int i = 0; i < TG; i++) z += red[i][e / CV_SITES][e % CV_SITES];
+    return z;
+  }
+};
+typedef Conv<SG_NF, SG_NC, false, SG_NT> Conv1;   // waves 11
+typedef Conv<SG_NC, SG_NC, false, 4> Conv2;       // 4
+typedef Conv<SG_NC, SG_NC, true, 4> Back1;        // 4
+typedef Conv<SG_NF, SG_NC, true, 2> Back0;        // 10
 
 // h1 = tanh(b1 + conv(W1, phi))
-__global__ void __launch_bounds__(SGB)
+__global__ void __launch_bounds__(Conv1::threads)
 k_sg_conv1(const unsigned short *__restrict__ wbf, const float *__restrict__ theta,
            const float *__restrict__ phi, const int *__restrict__ nbr, float *__restrict__ h1,
            int V) {
-  const int s = blockIdx.x * SGB + threadIdx.x;
-  if (s >= V) return;
-  float z[SG_NC];
-  conv_site<SG_NF, SG_NC, false>(wbf + SG_W1, phi, nbr, s, V, z);
-#pragma unroll
-  for (int o = 0; o < SG_NC; o++) ST(h1[(size_t)o * V + s], tanhf(z[o] + theta[SG_B1 + o]));
+  __shared__ Conv1 cv;
+  const int s0 = blockIdx.x * CV_SITES;
+  cv.run(wbf + SG_W1, phi, nbr, s0, V);
+  for (int e = threadIdx.x; e < SG_NC * CV_SITES; e += Conv1::threads) {
+    const int o = e / CV_SITES, s = s0 + e % CV_SITES;
+    if (s < V) ST(h1[(size_t)o * V + s], tanhf(cv.at(e) + theta[SG_B1 + o]));
+  }
 }
 
 // h2 = tanh(b2 + conv(W2, h1)); gz2 = (1 - h2^2) w3; partial of sum w3 . h2
-__global__ void __launch_bounds__(SGB)
+__global__ void __launch_bounds__(Conv2::threads)
 k_sg_conv2(const unsigned short *__restrict__ wbf, const float *__restrict__ theta,
            const float *__restrict__ h1, const int *__restrict__ nbr, float *__restrict__ h2,
            float *__restrict__ gz2, double *__restrict__ partial, int V) {
-  const int s = blockIdx.x * SGB + threadIdx.x;
+  __shared__ Conv2 cv;
+  const int s0 = blockIdx.x * CV_SITES;
+  cv.run(wbf + SG_W2, h1, nbr, s0, V);
   double act = 0;
-  if (s < V) {
-    float z[SG_NC];
-    conv_site<SG_NC, SG_NC, false>(wbf + SG_W2, h1, nbr, s, V, z);
-#pragma unroll
-    for (int o = 0; o < SG_NC; o++) {
-      const float h = tanhf(z[o] + theta[SG_B2 + o]), w = bf2f(wbf[SG_W3 + o]);
+  for (int e = threadIdx.x; e < SG_NC * CV_SITES; e += Conv2::threads) {
+    const int o = e / CV_SITES, s = s0 + e % CV_SITES;
+    if (s < V) {
+      const float h = tanhf(cv.at(e) + theta[SG_B2 + o]), w = bf2f(wbf[SG_W3 + o]);
       ST(h2[(size_t)o * V + s], h);
       ST(gz2[(size_t)o * V + s], (1.f - h * h) * w);
       act += (double)w * (double)h;
@@ -378,86 +445,97 @@ k_sg_conv2(const unsigned short *__restrict__ wbf, const float *__restrict__ the
 }
 
 // gz1 = (1 - h1^2) conv^T(W2, gz2)
-__global__ void __launch_bounds__(SGB)
+__global__ void __launch_bounds__(Back1::threads)
 k_sg_back1(const unsigned short *__restrict__ wbf, const float *__restrict__ gz2,
            const float *__restrict__ h1, const int *__restrict__ nbr, float *__restrict__ gz1,
            int V) {
-  const int s = blockIdx.x * SGB + threadIdx.x;
-  if (s >= V) return;
-  float g[SG_NC];
-  conv_site<SG_NC, SG_NC, true>(wbf + SG_W2, gz2, nbr, s, V, g);
-#pragma unroll
-  for (int i = 0; i < SG_NC; i++) {
-    const float h = h1[(size_t)i * V + s];
-    ST(gz1[(size_t)i * V + s], (1.f - h * h) * g[i]);
+  __shared__ Back1 cv;
+  const int s0 = blockIdx.x * CV_SITES;
+  cv.run(wbf + SG_W2, gz2, nbr, s0, V);
+  for (int e = threadIdx.x; e < SG_NC * CV_SITES; e += Back1::threads) {
+    const int i = e / CV_SITES, s = s0 + e % CV_SITES;
+    if (s < V) {
+      const float h = h1[(size_t)i * V + s];
+      ST(gz1[(size_t)i * V + s], (1.f - h * h) * cv.at(e));
+    }
   }
 }
 
 // gphi = conv^T(W1, gz1)
-__global__ void __launch_bounds__(SGB)
+__global__ void __launch_bounds__(Back0::threads)
 k_sg_back0(const unsigned short *__restrict__ wbf, const float *__restrict__ gz1,
            const int *__restrict__ nbr, float *__restrict__ gphi, int V) {
-  const int s = blockIdx.x * SGB + threadIdx.x;
-  if (s >= V) return;
-  float g[SG_NF];
-  conv_site<SG_NF, SG_NC, true>(wbf + SG_W1, gz1, nbr, s, V, g);
-#pragma unroll
-  for (int i = 0; i < SG_NF; i++) ST(gphi[(size_t)i * V + s], g[i]);
+  __shared__ Back0 cv;
+  const int s0 = blockIdx.x * CV_SITES;
+  cv.run(wbf + SG_W1, gz1, nbr, s0, V);
+  for (int e = threadIdx.x; e < SG_NF * CV_SITES; e += Back0::threads) {
+    const int i = e / CV_SITES, s = s0 + e % CV_SITES;
+    if (s < V) ST(gphi[(size_t)i * V + s], cv.at(e));
+  }
 }
 
-// F = dS/dUbar on link (x, a)
-__global__ void __launch_bounds__(SGB)
+// F = dS/dUbar on link (x, a).  A block makes one link direction of 16
+// sites: its 32 groups of 16 lanes take one of the link's 32 occurrences each,
+// whose contributions meet in the wave and then in LDS.  Large lattices are
+// bound by the links' lines that the XCDs' L2 miss, small ones by one
+// occurrence's chain of loads and products; a thread that owned a link made
+// its 32 of them one after the other (us: U(4) 4^3x8 269 -> 15, 8^3x16 325 ->
+// 166, 16^4 1542 -> 1368, U(2) 4^4 72 -> 6, 16^4 204 -> 206).  Four waves on 64
+// sites, eight occurrences each and no exchange between lanes, took 69, 213
+// and 1619 at the U(4) sizes.
+#define SGF_SITES 16
+#define SGF_THREADS (SGF_SITES * SG_NOCC)
+__global__ void __launch_bounds__(SGF_THREADS)
 k_sg_force(const double2 *__restrict__ U, const int *__restrict__ diff,
            const float *__restrict__ gphi, double2 *__restrict__ F, int V) {
-  const int x = blockIdx.x * SGB + threadIdx.x, a = blockIdx.y;
-  if (x >= V) return;
-  Mat acc;
-  mzero(acc);
+  __shared__ double2 part[SGF_THREADS / 64][NN][SGF_SITES];
+  int chunk, a;
+  if (!sg_block((V + SGF_SITES - 1) / SGF_SITES, NUMLINK, &chunk, &a)) return;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int col = threadIdx.x % SGF_SITES, o = threadIdx.x / SGF_SITES;
+  const int s0 = chunk * SGF_SITES, x = min(s0 + col, V - 1);
+  const int k = c_sg.ok[a][o], n = c_sg.nfac[k];
+  const int y = diff[c_sg.obase[a][o] * V + x];
+  const double sc = 0.5 / NCOL;
+  const bool dag = c_sg.fdag[k][c_sg.om[a][o]];
+  const double gr = sc * gphi[(size_t)(2 * k) * V + y],
+               gi = (dag ? -sc : sc) * gphi[(size_t)(2 * k + 1) * V + y];
+  Mat rest, f;
+  load_op(rest, U, c_sg.odir[a][o][0], diff[c_sg.odiff[a][o][0] * V + x], c_sg.odag[a][o][0], V);
 #pragma unroll 1
-  for (int o = 0; o < SG_NOCC; o++) {
-    const int k = c_sg.ok[a][o], n = c_sg.nfac[k];
-    const int y = diff[c_sg.obase[a][o] * V + x];
-    const double gr = gphi[(size_t)(2 * k) * V + y], gi = gphi[(size_t)(2 * k + 1) * V + y];
-    const double sc = 0.5 / NCOL;
-    Mat rest, f;
-    load_op(rest, U, c_sg.odir[a][o][0], diff[c_sg.odiff[a][o][0] * V + x], c_sg.odag[a][o][0],
-            V);
-#pragma unroll 1
-    for (int j = 1; j < n - 1; j++) {
-      load_op(f, U, c_sg.odir[a][o][j], diff[c_sg.odiff[a][o][j] * V + x], c_sg.odag[a][o][j],
-              V);
-      mmul_into(rest, f);
-    }
-    if (c_sg.fdag[k][c_sg.om[a][o]]) {
-      // conj(G) rest,  G = (gr + i gi) sc
-#pragma unroll
-      for (int i = 0; i < NCOL; i++)
-#pragma unroll
-        for (int j = 0; j < NCOL; j++) {
-          const double2 r = rest[i][j];
-          acc[i][j].x += sc * (gr * r.x + gi * r.y);
-          acc[i][j].y += sc * (gr * r.y - gi * r.x);
-        }
-    } else {
-      // G rest^dag
-#pragma unroll
-      for (int i = 0; i < NCOL; i++)
-#pragma unroll
-        for (int j = 0; j < NCOL; j++) {
-          const double2 r = make_double2(rest[j][i].x, -rest[j][i].y);
-          acc[i][j].x += sc * (gr * r.x - gi * r.y);
-          acc[i][j].y += sc * (gr * r.y + gi * r.x);
-        }
-    }
+  for (int j = 1; j < n - 1; j++) {
+    load_op(f, U, c_sg.odir[a][o][j], diff[c_sg.odiff[a][o][j] * V + x], c_sg.odag[a][o][j], V);
+    mmul_into(rest, f);
   }
-  const double gs = gphi[(size_t)(60 + a) * V + x] / (double)NCOL;
-  const double2 *u = U + (size_t)a * NN * V + x;
-  double2 *out = F + (size_t)a * NN * V + x;
 #pragma unroll
-  for (int e = 0; e < NN; e++) {
-    const double2 w = u[(size_t)e * V];
-    st_keep(out + (size_t)e * V, make_double2(acc[e / NCOL][e % NCOL].x + gs * w.x,
-                                              acc[e / NCOL][e % NCOL].y + gs * w.y));
+  for (int i = 0; i < NCOL; i++)
+#pragma unroll
+    for (int j = 0; j < NCOL; j++) {
+      // conj(G) rest where the loop holds U_a^dag, else G rest^dag,
+      // G = (gr + i gi) / (2N)
+      const double rx = dag ? rest[i][j].x : rest[j][i].x;
+      const double ry = dag ? rest[i][j].y : -rest[j][i].y;
+      double vx = gr * rx - gi * ry, vy = gr * ry + gi * rx;
+      for (int off = SGF_SITES; off < 64; off <<= 1) {
+        vx += __shfl_xor(vx, off, 64);
+        vy += __shfl_xor(vy, off, 64);
+      }
+      if ((i * NCOL + j) % (64 / SGF_SITES) == lane / SGF_SITES)
+        part[w][i * NCOL + j][col] = make_double2(vx, vy);
+    }
+  __syncthreads();
+  for (int q = threadIdx.x; q < NN * SGF_SITES; q += SGF_THREADS) {
+    const int e = q / SGF_SITES, s = s0 + q % SGF_SITES;
+    if (s >= V) continue;
+    const double gs = gphi[(size_t)(60 + a) * V + s] / (double)NCOL;
+    const double2 u = U[((size_t)a * NN + e) * V + s];
+    double2 t = make_double2(gs * u.x, gs * u.y);
+#pragma unroll
+    for (int i = 0; i < SGF_THREADS / 64; i++) {
+      t.x += part[i][e][q % SGF_SITES].x;
+      t.y += part[i][e][q % SGF_SITES].y;
+    }
+    st_keep(F + ((size_t)a * NN + e) * V + s, t);
   }
 }
 
@@ -490,58 +568,59 @@ k_sg_resid(const double2 *__restrict__ F, const double2 *__restrict__ Ft,
 }
 
 // tangent pass 1: z1d = conv(W1, v), h1d = (1 - h1^2) z1d
-__global__ void __launch_bounds__(SGB)
+__global__ void __launch_bounds__(Conv1::threads)
 k_sg_tan1(const unsigned short *__restrict__ wbf, const float *__restrict__ v,
           const float *__restrict__ h1, const int *__restrict__ nbr, float *__restrict__ z1d,
           float *__restrict__ h1d, int V) {
-  const int s = blockIdx.x * SGB + threadIdx.x;
-  if (s >= V) return;
-  float z[SG_NC];
-  conv_site<SG_NF, SG_NC, false>(wbf + SG_W1, v, nbr, s, V, z);
-#pragma unroll
-  for (int o = 0; o < SG_NC; o++) {
-    const float h = h1[(size_t)o * V + s];
-    ST(z1d[(size_t)o * V + s], z[o]);
-    ST(h1d[(size_t)o * V + s], (1.f - h * h) * z[o]);
+  __shared__ Conv1 cv;
+  const int s0 = blockIdx.x * CV_SITES;
+  cv.run(wbf + SG_W1, v, nbr, s0, V);
+  for (int e = threadIdx.x; e < SG_NC * CV_SITES; e += Conv1::threads) {
+    const int o = e / CV_SITES, s = s0 + e % CV_SITES;
+    if (s >= V) continue;
+    const float h = h1[(size_t)o * V + s], z = cv.at(e);
+    ST(z1d[(size_t)o * V + s], z);
+    ST(h1d[(size_t)o * V + s], (1.f - h * h) * z);
   }
 }
 
 // tangent pass 2: z2d = conv(W2, h1d); h2d = a2 z2d; adjoints
 // az2d = a2 w3, az2 = -2 h2 a2 w3 z2d  (a2 = 1 - h2^2)
-__global__ void __launch_bounds__(SGB)
+__global__ void __launch_bounds__(Conv2::threads)
 k_sg_tan2(const unsigned short *__restrict__ wbf, const float *__restrict__ h1d,
           const float *__restrict__ h2, const int *__restrict__ nbr, float *__restrict__ h2d,
           float *__restrict__ az2d, float *__restrict__ az2, int V) {
-  const int s = blockIdx.x * SGB + threadIdx.x;
-  if (s >= V) return;
-  float z[SG_NC];
-  conv_site<SG_NC, SG_NC, false>(wbf + SG_W2, h1d, nbr, s, V, z);
-#pragma unroll
-  for (int o = 0; o < SG_NC; o++) {
+  __shared__ Conv2 cv;
+  const int s0 = blockIdx.x * CV_SITES;
+  cv.run(wbf + SG_W2, h1d, nbr, s0, V);
+  for (int e = threadIdx.x; e < SG_NC * CV_SITES; e += Conv2::threads) {
+    const int o = e / CV_SITES, s = s0 + e % CV_SITES;
+    if (s >= V) continue;
     const float h = h2[(size_t)o * V + s], a2 = 1.f - h * h, w = bf2f(wbf[SG_W3 + o]);
-    ST(h2d[(size_t)o * V + s], a2 * z[o]);
+    const float z = cv.at(e);
+    ST(h2d[(size_t)o * V + s], a2 * z);
     ST(az2d[(size_t)o * V + s], a2 * w);
-    ST(az2[(size_t)o * V + s], -2.f * h * a2 * w * z[o]);
+    ST(az2[(size_t)o * V + s], -2.f * h * a2 * w * z);
   }
 }
 
 // tangent pass 3: ah1d = conv^T(W2, az2d); ah1 = conv^T(W2, az2) - 2 h1 ah1d z1d;
 // az1d = a1 ah1d, az1 = a1 ah1  (a1 = 1 - h1^2)
-__global__ void __launch_bounds__(SGB)
+__global__ void __launch_bounds__(Back1::threads)
 k_sg_tan3(const unsigned short *__restrict__ wbf, const float *__restrict__ az2d,
           const float *__restrict__ az2, const float *__restrict__ h1,
           const float *__restrict__ z1d, const int *__restrict__ nbr,
           float *__restrict__ az1d, float *__restrict__ az1, int V) {
-  const int s = blockIdx.x * SGB + threadIdx.x;
-  if (s >= V) return;
-  float gd[SG_NC], gp[SG_NC];
-  conv_site<SG_NC, SG_NC, true>(wbf + SG_W2, az2d, nbr, s, V, gd);
-  conv_site<SG_NC, SG_NC, true>(wbf + SG_W2, az2, nbr, s, V, gp);
-#pragma unroll
-  for (int i = 0; i < SG_NC; i++) {
-    const float h = h1[(size_t)i * V + s], a1 = 1.f - h * h;
-    const float ah1 = gp[i] - 2.f * h * gd[i] * z1d[(size_t)i * V + s];
-    ST(az1d[(size_t)i * V + s], a1 * gd[i]);
+  __shared__ Back1 gd, gp;
+  const int s0 = blockIdx.x * CV_SITES;
+  gd.run(wbf + SG_W2, az2d, nbr, s0, V);
+  gp.run(wbf + SG_W2, az2, nbr, s0, V);
+  for (int e = threadIdx.x; e < SG_NC * CV_SITES; e += Back1::threads) {
+    const int i = e / CV_SITES, s = s0 + e % CV_SITES;
+    if (s >= V) continue;
+    const float h = h1[(size_t)i * V + s], a1 = 1.f - h * h, d = gd.at(e);
+    const float ah1 = gp.at(e) - 2.f * h * d * z1d[(size_t)i * V + s];
+    ST(az1d[(size_t)i * V + s], a1 * d);
     ST(az1[(size_t)i * V + s], a1 * ah1);
   }
 }
@@ -788,22 +867,24 @@ extern "C" int susy_sg_get_params(susy_ctx *c, float *theta) {
 // `action` is non-null
 static int sg_eval(susy_ctx *c, const double2 *U, double *action) {
   SgState &S = *c->sg;
-  const int V = c->V, nb = (V + SGB - 1) / SGB;
-  hipLaunchKernelGGL(k_sg_features, dim3(nb), dim3(SGB), 0, c->s, U, S.d_base, S.phi, V);
-  hipLaunchKernelGGL(k_sg_conv1, dim3(nb), dim3(SGB), 0, c->s, S.wbf, S.theta, S.phi, c->d_nbr,
+  const int V = c->V, nc = (V + CV_SITES - 1) / CV_SITES;
+  hipLaunchKernelGGL(k_sg_features, dim3(sg_grid((V + SGF_B - 1) / SGF_B, SG_NLOOP + NUMLINK)),
+                     dim3(SGF_B), 0, c->s, U, S.d_base, S.phi, V);
+  hipLaunchKernelGGL(k_sg_conv1, dim3(nc), dim3(Conv1::threads), 0, c->s, S.wbf, S.theta, S.phi, c->d_nbr,
                      S.h1, V);
-  hipLaunchKernelGGL(k_sg_conv2, dim3(nb), dim3(SGB), 0, c->s, S.wbf, S.theta, S.h1, c->d_nbr,
+  hipLaunchKernelGGL(k_sg_conv2, dim3(nc), dim3(Conv2::threads), 0, c->s, S.wbf, S.theta, S.h1, c->d_nbr,
                      S.h2, S.gz2, c->d_part, V);
   HIPCHK(hipGetLastError());
   if (action) {
-    SGRET(reduce_partials(c, c->d_part, nb, 0));
+    SGRET(reduce_partials(c, c->d_part, nc, 0));
     SGRET(read_scalars(c, action, 1));
   }
-  hipLaunchKernelGGL(k_sg_back1, dim3(nb), dim3(SGB), 0, c->s, S.wbf, S.gz2, S.h1, c->d_nbr,
+  hipLaunchKernelGGL(k_sg_back1, dim3(nc), dim3(Back1::threads), 0, c->s, S.wbf, S.gz2, S.h1, c->d_nbr,
                      S.gz1, V);
-  hipLaunchKernelGGL(k_sg_back0, dim3(nb), dim3(SGB), 0, c->s, S.wbf, S.gz1, c->d_nbr, S.gphi,
+  hipLaunchKernelGGL(k_sg_back0, dim3(nc), dim3(Back0::threads), 0, c->s, S.wbf, S.gz1, c->d_nbr, S.gphi,
                      V);
-  hipLaunchKernelGGL(k_sg_force, dim3(nb, NUMLINK), dim3(SGB), 0, c->s, U, S.d_diff, S.gphi,
+  hipLaunchKernelGGL(k_sg_force, dim3(sg_grid((V + SGF_SITES - 1) / SGF_SITES, NUMLINK)),
+                     dim3(SGF_THREADS), 0, c->s, U, S.d_diff, S.gphi,
                      S.F, V);
   HIPCHK(hipGetLastError());
   return 0;
@@ -853,7 +934,7 @@ extern "C" int susy_sg_features(susy_ctx *c, float *phi) {
 static int sg_loss_grad(susy_ctx *c, const double2 *U, const double2 *Ft, double *loss,
                         bool grad, double gscale) {
   SgState &S = *c->sg;
-  const int V = c->V, nb = (V + SGB - 1) / SGB;
+  const int V = c->V, nc = (V + CV_SITES - 1) / CV_SITES;
   SGRET(sg_eval(c, U, nullptr));
   const size_t n = (size_t)NUMLINK * NN * V;
   const int rb = 256;
@@ -869,12 +950,13 @@ static int sg_loss_grad(susy_ctx *c, const double2 *U, const double2 *Ft, double
   }
   *loss = sc[0] / sc[1];
   if (!grad) return 0;
-  hipLaunchKernelGGL(k_sg_jvp, dim3(nb), dim3(SGB), 0, c->s, U, S.R, S.d_base, S.v, V);
-  hipLaunchKernelGGL(k_sg_tan1, dim3(nb), dim3(SGB), 0, c->s, S.wbf, S.v, S.h1, c->d_nbr, S.z1d,
+  hipLaunchKernelGGL(k_sg_jvp, dim3(sg_grid((V + SGF_B - 1) / SGF_B, SG_NLOOP + NUMLINK)),
+                     dim3(SGF_B), 0, c->s, U, S.R, S.d_base, S.v, V);
+  hipLaunchKernelGGL(k_sg_tan1, dim3(nc), dim3(Conv1::threads), 0, c->s, S.wbf, S.v, S.h1, c->d_nbr, S.z1d,
                      S.h1d, V);
-  hipLaunchKernelGGL(k_sg_tan2, dim3(nb), dim3(SGB), 0, c->s, S.wbf, S.h1d, S.h2, c->d_nbr,
+  hipLaunchKernelGGL(k_sg_tan2, dim3(nc), dim3(Conv2::threads), 0, c->s, S.wbf, S.h1d, S.h2, c->d_nbr,
                      S.h2d, S.az2d, S.az2, V);
-  hipLaunchKernelGGL(k_sg_tan3, dim3(nb), dim3(SGB), 0, c->s, S.wbf, S.az2d, S.az2, S.h1, S.z1d,
+  hipLaunchKernelGGL(k_sg_tan3, dim3(nc), dim3(Back1::threads), 0, c->s, S.wbf, S.az2d, S.az2, S.h1, S.z1d,
                      c->d_nbr, S.az1d, S.az1, V);
   SgGradIn in = {S.phi, S.v, S.h1, S.h1d, S.h2d, S.az2d, S.az2, S.az1d, S.az1};
   const int nchunk = (V + WG_CHUNK - 1) / WG_CHUNK;
