@@ -2,7 +2,7 @@
 // (reference: 4d_Q16/susy/congrad_multi.c:26-221), zero initial guess.
 //
 // The scalar recurrences (beta, zeta, alpha, convergence) are the reference's,
-// in FP64 on the host, so iteration counts follow the reference exactly.
+// in FP64, so iteration counts follow the reference exactly.
 // The vector work is restructured for HBM bandwidth:
 //   * D^dag D p0, + sigma_0 p0 and the <p0, A p0> partial sums are one
 //     operator pair with a fused epilogue;
@@ -16,7 +16,7 @@
 //     of the ring:
 //       p_j   = A_j p_j(k0)        + sum_l C_jl r_l
 //       psi_j = psi_j(k0) + E_j p_j(k0) + sum_l D_jl r_l
-//     with scalar coefficients advanced on the host by the same recurrences
+//     with scalar coefficients advanced by the same recurrences
 //     (zeta_0 = 1 for the base system, whose p0(k0) is kept by writing p0
 //     into the second of two buffers during the window); one fused flush
 //     applies them to all active systems every m iterations.
@@ -28,6 +28,7 @@
 //     sigma_0) psi_0 is recomputed with the FP64 operator and replaces r
 //     (the shifted residuals stay zeta_j r by construction).
 #include <math.h>
+#include <stddef.h>
 #include <stdio.h>
 #include <string.h>
 
@@ -53,7 +54,7 @@ __device__ __forceinline__ float2 from64<float2>(double2 v) {
   return make_float2((float)v.x, (float)v.y);
 }
 
-__device__ __forceinline__ void cg_block_sum(double v, double *partial) {
+__device__ __forceinline__ void cg_block_sum(double v, double *partial, int block) {
   for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
   __shared__ double red[CB / 64];
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
@@ -61,9 +62,50 @@ __device__ __forceinline__ void cg_block_sum(double v, double *partial) {
   if (threadIdx.x == 0) {
     double t = 0;
     for (int w = 0; w < CB / 64; w++) t += red[w];
-    partial[blockIdx.x] = t;
+    partial[block] = t;
     hold(t);
   }
+}
+
+// Sum of n partials, the same on every thread of a block of BS threads: a
+// fixed order with Neumaier compensation, so every block that makes the sum
+// gets the same bits.  One call a kernel: nothing guards its LDS against a second.
+template <int BS>
+__device__ __forceinline__ double cg_total(const double *__restrict__ part, int n) {
+  double s = 0, comp = 0;
+  auto add = [&](double v) {
+    const double t = s + v;
+    comp += (fabs(s) >= fabs(v)) ? (s - t) + v : (v - t) + s;
+    s = t;
+  };
+  for (int i0 = 0; i0 < n; i0 += 8 * BS) {
+    double v[8];
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+      const int i = i0 + k * BS + (int)threadIdx.x;
+      v[k] = i < n ? part[i] : 0.0;
+    }
+#pragma unroll
+    for (int k = 0; k < 8; k++) add(v[k]);
+  }
+  for (int off = 32; off > 0; off >>= 1) {
+    const double v = __shfl_xor(s, off, 64), c = __shfl_xor(comp, off, 64);
+    comp += c;
+    add(v);
+  }
+  __shared__ double rs[BS / 64], rc[BS / 64];
+  if ((threadIdx.x & 63) == 0) {
+    rs[threadIdx.x >> 6] = s;
+    rc[threadIdx.x >> 6] = comp;
+  }
+  __syncthreads();
+  s = rs[0];
+  comp = rc[0];
+  for (int w = 1; w < BS / 64; w++) {
+    comp += rc[w];
+    add(rs[w]);
+  }
+  return s + comp;
 }
 
 struct PsiPtrs {
@@ -86,16 +128,21 @@ k_cg_init(const double2 *__restrict__ src, C *__restrict__ r, C *__restrict__ p0
     for (int j = 0; j < nsh; j++) st_keep(psi.p[j] + i, make_double2(0, 0));
     s += v.x * v.x + v.y * v.y;
   }
-  cg_block_sum(s, partial);
+  cg_block_sum(s, partial, blockIdx.x);
 }
 
 // Scalar state of one solve, in device memory.  The reference's recurrences
-// (congrad_multi.c:60-180) run in single-thread kernels between the vector
-// passes, so the host enqueues iterations without waiting for them; a
-// solver that has converged turns every queued launch into a no-op.
+// (congrad_multi.c:60-180) run between the vector passes, so the host enqueues
+// iterations without waiting for them; a solver that has converged turns
+// every queued launch into a no-op.
+//
+// done and rsq have two slots: an iteration reads slot par (the parity of the
+// iterations queued before it) and its p update, the last pass, writes the
+// other one.  Blocks of that pass may then make alpha_0 themselves while one
+// of them advances the state.
 struct CgState {
-  int done, iteration;          // read back by the host (first 24 bytes)
-  double rsq, rsqstop;
+  int done[2], iteration;       // read back by the host (first 40 bytes)
+  double rsq[2], rsqstop;
   int skip_rel, maxcg, nsh, cnt;
   double shifts[MAXSH];
   double zi[MAXSH], zim1[MAXSH], zip1[MAXSH], bi[MAXSH], bim1[MAXSH], al[MAXSH];
@@ -129,138 +176,153 @@ k_cgs_init(CgState *st, const double *__restrict__ source_norm, double errormin,
   if (threadIdx.x == 0) {
     const double rsq = *source_norm;
     const double stop = errormin * rsq;
-    st->rsq = rsq;
+    st->rsq[0] = rsq;
     st->rsqstop = stop;
     st->iteration = 0;
     st->maxcg = maxcg;
     st->nsh = nsh;
     st->cnt = 0;
-    st->done = !(0 < maxcg && rsq > stop);
+    st->done[0] = !(0 < maxcg && rsq > stop);
     st->skip_rel = 0;
     hold(rsq);
     hold(stop);
   }
 }
 
-// the while condition of the iteration loop, evaluated at the end of each
-// iteration (after its p update, which the converged iteration still makes):
-// everything queued after it -- flushes, reliable updates, further
-// iterations -- then sees the solve finished
-__global__ void k_cgs_stop(CgState *st) {
-  if (!st->done && !(st->iteration < st->maxcg && st->rsq > st->rsqstop)) st->done = 1;
-}
-
-// beta and the shifted zeta / beta after A p0 and <p0, A p0> = *cd
-__global__ void k_cgs_beta(CgState *st, const double *__restrict__ cd) {
+// beta and the shifted zeta / beta after A p0 and <p0, A p0> = cd, by the
+// threads j < nsh of one block (the threads from MAXSH on do nothing here)
+__device__ __forceinline__ void cgs_beta(CgState *st, double cd, int par) {
 #pragma clang fp contract(off)
-  if (st->done) return;
+  const int j = threadIdx.x;
+  if (j >= MAXSH) return;
   // every load before the first store (vm_drain: see its definition)
-  const int it = st->iteration, nsh = st->nsh;
-  const double rsq = st->rsq, cdv = *cd, al0 = st->al[0], bim10 = st->bim1[0],
-               s0 = st->shifts[0];
+  const int it = st->iteration, nsh = st->nsh, cv = st->conv[j];
+  const double rsq = st->rsq[par], al0 = st->al[0], bim10 = st->bim1[0], s0 = st->shifts[0];
+  const double zij = st->zi[j], zim1j = st->zim1[j], sj = st->shifts[j];
   vm_drain();
-  const double bi0 = -rsq / cdv;
-  st_keep(&st->iteration, it + 1);
-  st->bi[0] = bi0;
-  hold(bi0);
-  st_keep(&st->zip1[0], 1.0);
-  for (int j = 1; j < nsh; j++) {
-    const int cv = st->conv[j];
-    const double zij = st->zi[j], zim1j = st->zim1[j], sj = st->shifts[j];
-    vm_drain();
-    if (cv) continue;
-    double zp = zij * zim1j * bim10;
-    const double c1 = bi0 * al0 * (zim1j - zij);
-    const double c2 = zim1j * bim10 * (1 - (sj - s0) * bi0);
-    zp /= c1 + c2;
-    const double bj = bi0 * zp / zij;
-    st->zip1[j] = zp;
-    st->bi[j] = bj;
-    hold(zp);
-    hold(bj);
+  const double bi0 = -rsq / cd;
+  if (j == 0) {
+    st_keep(&st->iteration, it + 1);
+    st_keep(&st->bi[0], bi0);
+    st_keep(&st->zip1[0], 1.0);
+    return;
   }
+  if (j >= nsh || cv) return;
+  double zp = zij * zim1j * bim10;
+  const double c1 = bi0 * al0 * (zim1j - zij);
+  const double c2 = zim1j * bim10 * (1 - (sj - s0) * bi0);
+  zp /= c1 + c2;
+  const double bj = bi0 * zp / zij;
+  st_keep(&st->zip1[j], zp);
+  st_keep(&st->bi[j], bj);
 }
 
 // alpha, the window coefficients, convergence of the shifted systems and the
-// advance of the recurrences after |r_new|^2 = *rsqnew.  One block of
-// MAXSH x MAXWIN threads: thread (j, l) updates the window coefficients
-// Cw[j][l], Dw[j][l]; thread l = 0 of shift j does that shift's scalars.
-// Every element sees the same operations in the same order as a serial
-// loop over j and l would make.
-#define ALPHA_THREADS (MAXSH * MAXWIN)
-__global__ void __launch_bounds__(ALPHA_THREADS)
-k_cgs_alpha(CgState *st, const double *__restrict__ rsqnew) {
+// advance of the recurrences after |r_new|^2 = rn, by one block of BS threads:
+// thread (j, l) updates the window coefficients Cw[j][l], Dw[j][l]; thread
+// l = 0 of shift j does that shift's scalars.  Every element sees the same
+// operations in the same order as a serial loop over j and l would make.
+// Last, the while condition of the iteration loop: the converged iteration
+// still makes its p update, and everything queued after it -- flushes,
+// reliable updates, further iterations -- sees the solve finished.
+template <int BS>
+__device__ __forceinline__ void cgs_alpha(CgState *st, double rn, int par) {
 #pragma clang fp contract(off)
-  if (st->done) return;
   __shared__ double al_s[MAXSH], bi_s[MAXSH];
   __shared__ int conv_s[MAXSH];
-  const int j = threadIdx.x / MAXWIN, l = threadIdx.x % MAXWIN;
+  constexpr int NW = MAXSH * MAXWIN / BS;   // window coefficients per thread
+  static_assert(NW * BS == MAXSH * MAXWIN && BS >= MAXSH, "threads of the state's block");
   // every load before the first store (vm_drain: see its definition)
-  const int nsh = st->nsh, cnt = st->cnt;
-  const double rn = *rsqnew, rsq = st->rsq, rsqstop = st->rsqstop;
-  const bool lead = l == 0 && j < nsh;
+  const int nsh = st->nsh, cnt = st->cnt, it = st->iteration, maxcg = st->maxcg;
+  const double rsq = st->rsq[par], rsqstop = st->rsqstop;
+  const int js = threadIdx.x;               // the shift whose scalars this thread does
+  const bool lead = js < nsh;
   int cv = 0;
-  double zij = 0, zp1 = 0, bij = 0, bi0 = 0, alj = 0, Ej = 0, Aj = 0, cw = 0, dw = 0;
+  double zij = 0, zp1 = 0, bij = 0, bi0 = 0, alj = 0, Ej = 0, Aj = 0, cw[NW], dw[NW];
   if (lead) {
-    cv = st->conv[j];
-    zij = st->zi[j];
-    zp1 = st->zip1[j];
-    bij = st->bi[j];
+    cv = st->conv[js];
+    zij = st->zi[js];
+    zp1 = st->zip1[js];
+    bij = st->bi[js];
     bi0 = st->bi[0];
-    alj = st->al[j];
-    Ej = st->E[j];
-    Aj = st->A[j];
+    alj = st->al[js];
+    Ej = st->E[js];
+    Aj = st->A[js];
   }
-  if (j < nsh && l < cnt) {
-    cw = st->Cw[j][l];
-    dw = st->Dw[j][l];
+#pragma unroll
+  for (int m = 0; m < NW; m++) {
+    const int e = threadIdx.x + m * BS, j = e / MAXWIN, l = e % MAXWIN;
+    cw[m] = dw[m] = 0;
+    if (j < nsh && l < cnt) {
+      cw[m] = st->Cw[j][l];
+      dw[m] = st->Dw[j][l];
+    }
   }
   vm_drain();
   if (lead) {
     const double a0 = rn / rsq;
-    if (j == 0) alj = a0;
+    if (js == 0) alj = a0;
     else if (!cv) alj = a0 * zp1 * bij / (zij * bi0);
-    al_s[j] = alj;
-    bi_s[j] = bij;
-    conv_s[j] = cv;
+    al_s[js] = alj;
+    bi_s[js] = bij;
+    conv_s[js] = cv;
   }
   __syncthreads();
-  if (j < nsh && !conv_s[j]) {
-    // psi_j -= beta_j p_j, then p_j = zeta_j r + alpha_j p_j (zeta_0 = 1)
-    if (l < cnt) {
-      const double d2 = dw - bi_s[j] * cw, c2 = cw * al_s[j];
-      st->Dw[j][l] = d2;
-      st->Cw[j][l] = c2;
-      hold(d2);
-      hold(c2);
-    }
-    if (l == 0) {
-      const double e2 = Ej - bij * Aj, a2 = Aj * alj;
-      st->al[j] = alj;
-      st->touched[j] = 1;
-      st->E[j] = e2;
-      st->A[j] = a2;
-      st->Cw[j][cnt] = zp1;
-      hold(e2);
-      hold(a2);
-    }
+  // psi_j -= beta_j p_j, then p_j = zeta_j r + alpha_j p_j (zeta_0 = 1)
+#pragma unroll
+  for (int m = 0; m < NW; m++) {
+    const int e = threadIdx.x + m * BS, j = e / MAXWIN, l = e % MAXWIN;
+    if (j >= nsh || conv_s[j] || l >= cnt) continue;
+    const double d2 = dw[m] - bi_s[j] * cw[m], c2 = cw[m] * al_s[j];
+    st_keep(&st->Dw[j][l], d2);
+    st_keep(&st->Cw[j][l], c2);
   }
-  if (lead) {
-    int c2 = cv;
-    if (j > 0 && !cv && rn * zp1 * zp1 <= rsqstop) {
-      c2 = 1;
-      st->conv[j] = 1;
-    }
-    if (!c2) {
-      st->bim1[j] = bij;
-      st->zim1[j] = zij;
-      st->zi[j] = zp1;
+  if (lead && !cv) {
+    const double e2 = Ej - bij * Aj, a2 = Aj * alj;
+    st_keep(&st->al[js], alj);
+    st_keep(&st->touched[js], 1);
+    st_keep(&st->E[js], e2);
+    st_keep(&st->A[js], a2);
+    st_keep(&st->Cw[js][cnt], zp1);
+    if (js > 0 && rn * zp1 * zp1 <= rsqstop) {
+      st_keep(&st->conv[js], 1);
+    } else {
+      st_keep(&st->bim1[js], bij);
+      st_keep(&st->zim1[js], zij);
+      st_keep(&st->zi[js], zp1);
     }
   }
   if (threadIdx.x == 0) {
-    st->cnt = cnt + 1;
-    st->rsq = rn;
+    st_keep(&st->cnt, cnt + 1);
+    st_keep(&st->rsq[par ^ 1], rn);
+    st_keep(&st->done[par ^ 1], (int)!(it < maxcg && rn > rsqstop));
   }
+}
+
+// an idle iteration hands its slot of the state on
+__device__ __forceinline__ void cgs_idle(CgState *st, int par) {
+  if (threadIdx.x == 0) {
+    const double rsq = st->rsq[par];
+    st_keep(&st->rsq[par ^ 1], rsq);
+    st_keep(&st->done[par ^ 1], 1);
+  }
+}
+
+// The two scalar steps as launches of one block, for lattices with more
+// partials than the blocks of the vector passes should each sum.
+#define CGS_THREADS (MAXSH * MAXWIN)
+__global__ void __launch_bounds__(CGS_THREADS)
+k_cgs_beta(CgState *st, const double *__restrict__ part, int n, int par) {
+  if (st->done[par]) return;
+  cgs_beta(st, cg_total<CGS_THREADS>(part, n), par);
+}
+__global__ void __launch_bounds__(CGS_THREADS)
+k_cgs_alpha(CgState *st, const double *__restrict__ part, int n, int par) {
+  if (st->done[par]) {
+    cgs_idle(st, par);
+    return;
+  }
+  cgs_alpha<CGS_THREADS>(st, cg_total<CGS_THREADS>(part, n), par);
 }
 
 // window state after a flush (MAXSH x MAXWIN threads)
@@ -281,27 +343,40 @@ k_cgs_reset(CgState *st, const int *__restrict__ skip) {
 }
 
 // the reliable update runs only while the solve is open and unconverged
-__global__ void k_cgs_relcheck(CgState *st) {
-  st->skip_rel = st->done || !(st->rsq > st->rsqstop);
+__global__ void k_cgs_relcheck(CgState *st, int par) {
+  st->skip_rel = st->done[par] || !(st->rsq[par] > st->rsqstop);
 }
 __global__ void k_cgs_setrsq(CgState *st, const double *__restrict__ v,
-                             const int *__restrict__ skip) {
+                             const int *__restrict__ skip, int par) {
   if (skip != nullptr && *skip) return;
-  st->rsq = *v;
+  st->rsq[par] = *v;
 }
-__global__ void k_cgs_reopen(CgState *st) { st->done = 0; }
+__global__ void k_cgs_reopen(CgState *st, int par) { st->done[par] = 0; }
 
 // rout = rin + beta_0 * ap; partial |rout|^2.  rout is the next slot of the
 // residual window and rin the previous one (the same slot when the window
 // holds one residual: the update is elementwise, so in place is safe).
-template <typename C>
+// SUM: every block makes beta_0 from the ndot partials of <p0, A p0>, and
+// block 0 advances the state beside them; else k_cgs_beta ran before.
+template <typename C, bool SUM>
 __global__ void __launch_bounds__(CB)
-k_cg_r(const C *rin, const C *__restrict__ ap, C *rout, const CgState *__restrict__ st,
-       size_t n, double *__restrict__ partial) {
-  if (st->done) return;
-  const double beta0 = st->bi[0];
+k_cg_r(const C *rin, const C *__restrict__ ap, C *rout, CgState *st, size_t n,
+       const double *__restrict__ dot, int ndot, double *__restrict__ partial, int par) {
+  if (st->done[par]) return;
+  const int nb = SUM ? gridDim.x - 1 : gridDim.x, b = SUM ? (int)blockIdx.x - 1 : blockIdx.x;
+  double beta0;
+  if (SUM) {
+    const double cd = cg_total<CB>(dot, ndot);
+    if (b < 0) {
+      cgs_beta(st, cd, par);
+      return;
+    }
+    beta0 = -st->rsq[par] / cd;
+  } else {
+    beta0 = st->bi[0];
+  }
   double s = 0;
-  for (size_t i = (size_t)blockIdx.x * CB + threadIdx.x; i < n; i += (size_t)gridDim.x * CB) {
+  for (size_t i = (size_t)b * CB + threadIdx.x; i < n; i += (size_t)nb * CB) {
     C a = ap[i], v = rin[i];
     vm_drain();   // loads of this element complete before its store
     v.x = fma(beta0, a.x, v.x);
@@ -309,26 +384,43 @@ k_cg_r(const C *rin, const C *__restrict__ ap, C *rout, const CgState *__restric
     st_keep(rout + i, v);
     s += (double)v.x * (double)v.x + (double)v.y * (double)v.y;
   }
-  cg_block_sum(s, partial);
+  cg_block_sum(s, partial, b);
 }
 
 // pout = r + alpha_0 pin (pout is pin, or the other p0 buffer at the first
 // iteration of a window, which leaves the window-start p0 intact), one thread
 // per (site, Twist_Fermion component); the thread also stores the
 // operator's pre-pass values of the new p for the next D:
-// aux[0] = Tr p_0, aux[1+a] = Tr(U_a^-1 p_{1+a}) (aux = nullptr: no G terms)
+// aux[0] = Tr p_0, aux[1+a] = Tr(U_a^-1 p_{1+a}) (aux = nullptr: no G terms).
+// SUM: every block makes alpha_0 from the nrsq partials of |r|^2, and a block of
+// the first row advances the state beside them; else k_cgs_alpha ran before.
 template <typename C> struct ScalarOf;
 template <> struct ScalarOf<float2> { typedef float t; };
 template <> struct ScalarOf<double2> { typedef double t; };
-template <typename C>
+template <typename C, bool SUM>
 __global__ void __launch_bounds__(CB)
 k_cg_p0_prep(const C *pin, const C *__restrict__ r, C *pout, const C *__restrict__ uinv,
-             C *__restrict__ aux, const CgState *__restrict__ st, int V) {
+             C *__restrict__ aux, CgState *st, int V, const double *__restrict__ part, int nrsq,
+             int par) {
   typedef typename ScalarOf<C>::t R;
-  if (st->done) return;
-  const int s = blockIdx.x * CB + threadIdx.x, k = blockIdx.y;
+  const int s = blockIdx.x * CB + threadIdx.x, k = SUM ? (int)blockIdx.y - 1 : blockIdx.y;
+  if (st->done[par]) {
+    if (SUM && k < 0 && blockIdx.x == 0) cgs_idle(st, par);
+    return;
+  }
+  double alpha0;
+  if (SUM) {
+    if (k < 0 && blockIdx.x > 0) return;
+    const double rn = cg_total<CB>(part, nrsq);
+    if (k < 0) {
+      cgs_alpha<CB>(st, rn, par);
+      return;
+    }
+    alpha0 = rn / st->rsq[par];
+  } else {
+    alpha0 = st->al[0];
+  }
   if (s >= V) return;
-  const double alpha0 = st->al[0];
   const bool pre = aux != nullptr && k <= NUMLINK;
   // every load before the first store (vm_drain: see its definition)
   C v[NN], rv[NN], u[NN];
@@ -437,7 +529,7 @@ k_true_res(const double2 *__restrict__ src, const double2 *__restrict__ ap,
     st_keep(r + i, from64<C>(v));
     s += v.x * v.x + v.y * v.y;
   }
-  cg_block_sum(s, partial);
+  cg_block_sum(s, partial, blockIdx.x);
 }
 
 // ---------------------------------------------------------------------
@@ -465,6 +557,18 @@ extern "C" int susy_set_cg_options(int window, int reliable) {
   return 0;
 }
 
+// Partials of <p0, A p0> up to which every block of the two vector passes sums
+// them itself and one block beside them advances the scalar state: an
+// iteration is then four launches, where k_cgs_beta and k_cgs_alpha make it
+// six (and a launch per reduction, recurrence and stopping test made it nine).
+// Above, the blocks' sums cost more than the two launches.  us of an
+// iteration, nine | six | four launches:
+//   U(2) 4^4 FP64 31.1 | 26.4 | 22.1       U(3) 4^4 FP32 32.2 | 27.5 | 22.3
+//   U(4) 4^3x8 FP32 38.8 | 32.8 | 28.7     U(4) 8^3x16 FP32 117.1 | 110.2 | 107.3
+//   U(2) 8^2x16^2 FP64 91.7 | 83.8 | 81.0  U(2) 16^4 FP32 201.8 | 199.4 | 202.2
+//   U(2) 16^3x32 FP32 (32768 partials) 394 | 386 | 396
+#define CG_SUM_PARTS 8192
+
 // iterations enqueued between two read-backs of the solver status
 #define CG_BATCH 16
 
@@ -490,7 +594,9 @@ static int cg_impl(susy_ctx *c, const double2 *src, double2 *const *psim, int ns
   }
   if (!c->cg_state) HIPCHK(hipMalloc(&c->cg_state, sizeof(CgState)));
   CgState *st = (CgState *)c->cg_state;
-  const int *d_done = &st->done, *d_skiprel = &st->skip_rel;
+  const int *d_skiprel = &st->skip_rel;
+  // parity of the iterations queued so far: the current slot of done and rsq
+  int par = 0;
   C *base = (C *)c->cg_ws;
   C *p0buf[2] = {base, base + n};
   C *ap = base + 2 * n, *tmp = base + 3 * n;
@@ -506,8 +612,10 @@ static int cg_impl(susy_ctx *c, const double2 *src, double2 *const *psim, int ns
   PsiPtrs psi;
   for (int j = 0; j < nsh; j++) psi.p[j] = psim[j];
   double sigma0 = shifts[0] + ((c->p.fmass > IMAG_TOL) ? c->p.fmass * c->p.fmass : 0.0);
-  double *d_norm = c->d_scal, *d_cd = c->d_scal + 1, *d_rn = c->d_scal + 2,
-         *d_true = c->d_scal + 3;
+  double *d_norm = c->d_scal, *d_true = c->d_scal + 3;
+  // partials of |r|^2, apart from those of <p0, A p0>, which other blocks of
+  // the r update may still read
+  double *part_r = c->d_part + c->npart;
 
   // Host bookkeeping of the buffers, a function of the iteration count: r is
   // the newest window slot (before the first iteration the last one), pcur
@@ -536,8 +644,8 @@ static int cg_impl(susy_ctx *c, const double2 *src, double2 *const *psim, int ns
                      shv, MaxCG);
   HIPCHK(hipGetLastError());
 
-  auto one = [&](void (*k)(CgState *)) -> int {
-    hipLaunchKernelGGL(k, dim3(1), dim3(1), 0, c->s, st);
+  auto one = [&](void (*k)(CgState *, int)) -> int {
+    hipLaunchKernelGGL(k, dim3(1), dim3(1), 0, c->s, st, par);
     HIPCHK(hipGetLastError());
     return 0;
   };
@@ -566,10 +674,10 @@ static int cg_impl(susy_ctx *c, const double2 *src, double2 *const *psim, int ns
     int r1, nbd = 0;
     if (fp32) {
       r1 = dsq_pair32(c, (const float2 *)in, (float2 *)tmp, (float2 *)out, (float)sigma0,
-                      c->d_part, &nbd, d_done, !in_prepped);
+                      c->d_part, &nbd, &st->done[par], !in_prepped);
     } else {
       r1 = dsq_pair64(c, (const double2 *)in, (double2 *)tmp, (double2 *)out, sigma0,
-                      c->d_part, &nbd, d_done, !in_prepped);
+                      c->d_part, &nbd, &st->done[par], !in_prepped);
     }
     *nbo = nbd;
     return r1;
@@ -585,7 +693,7 @@ static int cg_impl(susy_ctx *c, const double2 *src, double2 *const *psim, int ns
                        skip);
     HIPCHK(hipGetLastError());
     if ((r1 = reduce_partials(c, c->d_part, nb, 3))) return r1;
-    hipLaunchKernelGGL(k_cgs_setrsq, dim3(1), dim3(1), 0, c->s, st, d_true, skip);
+    hipLaunchKernelGGL(k_cgs_setrsq, dim3(1), dim3(1), 0, c->s, st, d_true, skip, par);
     HIPCHK(hipGetLastError());
     return 0;
   };
@@ -593,10 +701,13 @@ static int cg_impl(susy_ctx *c, const double2 *src, double2 *const *psim, int ns
     int done, iteration;
     double rsq, rsqstop;
   } stat = {0, 0, 0.0, 0.0};
+  constexpr size_t head = offsetof(CgState, skip_rel);
   auto read_status = [&]() -> int {
-    HIPCHK(hipMemcpyAsync(c->h_scal, st, sizeof(Status), hipMemcpyDeviceToHost, c->s));
+    HIPCHK(hipMemcpyAsync(c->h_scal, st, head, hipMemcpyDeviceToHost, c->s));
     HIPCHK(hipStreamSynchronize(c->s));
-    memcpy(&stat, c->h_scal, sizeof(Status));
+    CgState h;
+    memcpy(&h, c->h_scal, head);
+    stat = {h.done[par], h.iteration, h.rsq[par], h.rsqstop};
     return 0;
   };
 
@@ -613,27 +724,35 @@ static int cg_impl(susy_ctx *c, const double2 *src, double2 *const *psim, int ns
       for (int k = 0; k < CG_BATCH; k++) {
         int nbd;
         if ((e = dsq(pcur, ap, &nbd, p_prepped))) return e;
-        if ((e = reduce_partials(c, c->d_part, nbd, 1))) return e;
-        hipLaunchKernelGGL(k_cgs_beta, dim3(1), dim3(1), 0, c->s, st, d_cd);
+        const bool sum = nbd <= CG_SUM_PARTS;
         C *rnew = slot(host_cnt);
-        hipLaunchKernelGGL((k_cg_r<C>), dim3(nb), dim3(CB), 0, c->s, r, ap, rnew, st, n,
-                           c->d_part);
-        HIPCHK(hipGetLastError());
-        if ((e = reduce_partials(c, c->d_part, nb, 2))) return e;
-        hipLaunchKernelGGL(k_cgs_alpha, dim3(1), dim3(ALPHA_THREADS), 0, c->s, st, d_rn);
         C *pnext = pcur != pfrozen ? pcur : (pcur == p0buf[0] ? p0buf[1] : p0buf[0]);
-        hipLaunchKernelGGL((k_cg_p0_prep<C>), dim3((c->V + CB - 1) / CB, NTF), dim3(CB), 0, c->s,
-                           pcur, rnew, pnext, uinv_c, aux_c, st, c->V);
+        const unsigned nbp = (c->V + CB - 1) / CB;
+        if (sum) {
+          hipLaunchKernelGGL((k_cg_r<C, true>), dim3(nb + 1), dim3(CB), 0, c->s, r, ap, rnew, st,
+                             n, c->d_part, nbd, part_r, par);
+          hipLaunchKernelGGL((k_cg_p0_prep<C, true>), dim3(nbp, NTF + 1), dim3(CB), 0, c->s, pcur,
+                             rnew, pnext, uinv_c, aux_c, st, c->V, part_r, nb, par);
+        } else {
+          hipLaunchKernelGGL(k_cgs_beta, dim3(1), dim3(CGS_THREADS), 0, c->s, st, c->d_part, nbd,
+                             par);
+          hipLaunchKernelGGL((k_cg_r<C, false>), dim3(nb), dim3(CB), 0, c->s, r, ap, rnew, st, n,
+                             c->d_part, nbd, part_r, par);
+          hipLaunchKernelGGL(k_cgs_alpha, dim3(1), dim3(CGS_THREADS), 0, c->s, st, part_r, nb,
+                             par);
+          hipLaunchKernelGGL((k_cg_p0_prep<C, false>), dim3(nbp, NTF), dim3(CB), 0, c->s, pcur,
+                             rnew, pnext, uinv_c, aux_c, st, c->V, part_r, nb, par);
+        }
         HIPCHK(hipGetLastError());
+        par ^= 1;
         p_prepped = aux_c != nullptr;
         r = rnew;
         pcur = pnext;
         host_cnt++;
-        if ((e = one(k_cgs_stop))) return e;
         log[k] = {r, pcur, pfrozen};
         // window end: a solve that has finished keeps its open window for
         // the final flush below, made with the restored buffers
-        if (host_cnt == m && (e = flush(d_done))) return e;
+        if (host_cnt == m && (e = flush(&st->done[par]))) return e;
         if (fp32 && ++since_reliable >= g_reliable) {
           since_reliable = 0;
           if ((e = one(k_cgs_relcheck))) return e;

@@ -77,3 +77,37 @@ def test_surrogate_site_blocks(ncol, dims):
     assert abs(loss / loss_ref - 1) < 1e-5
     assert rel_err(g, sr.pack(g_ref).astype(np.float64)) < 1e-4
     lat.close()
+
+
+# The two ways of an iteration's scalar steps: blocks that sum up to 8192
+# partials themselves (the last size of it) and one block above.  The first 12
+# iterations follow the oracle to rounding (later ones amplify it: on the U(3)
+# lattice |r|^2 of any two roundings differs by 1e-5 after 40 and by a tenth
+# after 46); at the end every system's true residual is below the bound, with
+# the FP32 form's margin as in its other tests.
+@pytest.mark.parametrize("ncol,dims", [(2, (2, 2, 2, 2)), (3, (3, 3, 2, 5)), (2, (16, 16, 16, 8)),
+                                       (2, (16, 15, 18, 8))])
+def test_solver_scalar_steps(ncol, dims):
+    print("solver", ncol, dims, flush=True)
+    O, lat = pair(ncol, dims)
+    lk = random_links(O.link_shape(), 3, 0.2)
+    O.set_links(lk)
+    lat.set_links(lk)
+    src = random_tf(O.tf_shape(), 9)
+    shifts = [0.5, 2.0, 9.0]
+    h = lat.tf_alloc(5)
+    lat.tf_upload(h, src)
+    it, sz = lat.congrad_multi(h, h + 1, shifts, 12, 1e-10)
+    it_o, sz_o, psi = O.congrad_multi(src, shifts, 12, 1e-10)
+    assert it == it_o == 12
+    assert abs(sz / sz_o - 1) < 1e-6
+    for j in range(3):
+        assert rel_err(lat.tf_download(h + 1 + j), psi[j]) < 1e-10, j
+    n2 = np.vdot(src, src).real
+    for form, margin in ((susy_amd.FORM_FP64, 1.01), (susy_amd.FORM_FP32, 4)):
+        assert lat.congrad_multi(h, h + 1, shifts, 500, 1e-10, form)[0] < 500
+        for j in range(3):
+            lat.dsq(h + 1 + j, h + 4)
+            r = src - lat.tf_download(h + 4) - shifts[j] * lat.tf_download(h + 1 + j)
+            assert np.vdot(r, r).real <= margin * 1e-10 * n2, (form, j)
+    lat.close()
