@@ -190,7 +190,7 @@ static int ctx_setup(susy_ctx *c) {
   RET(dalloc(&c->f_links, mat5));
   RET(dalloc(&c->f_uinv, mat5));
   RET(dalloc(&c->f_pdet, (size_t)NUMLINK * NUMLINK * V));
-  RET(dalloc(&c->d_aux, (size_t)12 * V));
+  RET(dalloc(&c->d_aux, (size_t)6 * V));
   RET(dalloc(&c->f_aux, (size_t)6 * V));
   RET(dalloc(&c->d_aux2, (size_t)6 * V));
   RET(dalloc(&c->f_aux2, (size_t)6 * V));

@@ -25,7 +25,7 @@
 // contiguous slab of site chunks, all 16 component-blocks of a chunk back to
 // back: neighbouring chunks (the z and t neighbours of a site) then share the
 // same L2.
-#include "susy_internal.h"
+#include "dev_buf.h"
 
 #include <mutex>
 
@@ -66,33 +66,6 @@ int dslash_init_tables(const PlaqTerms &pt) {
 #define DS_STR(x) #x
 #define DS_UNROLL_LOOP(n) _Pragma(DS_STR(unroll n))
 
-template <typename C, typename R>
-__device__ __forceinline__ void cfma(C &acc, R ar, R ai, C b) {
-  acc.x = fma(ar, b.x, acc.x);
-  acc.x = fma(-ai, b.y, acc.x);
-  acc.y = fma(ar, b.y, acc.y);
-  acc.y = fma(ai, b.x, acc.y);
-}
-
-typedef __amdgpu_buffer_rsrc_t Rsrc;
-
-__device__ __forceinline__ Rsrc make_rsrc(const void *p, uint32_t bytes) {
-  // dword3 0x00020000: raw (untyped) access on the gfx9 family
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), (short)0, (int)bytes,
-                                           0x00020000);
-}
-template <typename C> __device__ __forceinline__ C bload(Rsrc r, uint32_t voff, uint32_t soff);
-template <>
-__device__ __forceinline__ double2 bload<double2>(Rsrc r, uint32_t voff, uint32_t soff) {
-  return __builtin_bit_cast(double2, __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0));
-}
-template <>
-__device__ __forceinline__ float2 bload<float2>(Rsrc r, uint32_t voff, uint32_t soff) {
-  return __builtin_bit_cast(float2, __builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, 0));
-}
-__device__ __forceinline__ int bload_i32(Rsrc r, uint32_t voff, uint32_t soff) {
-  return (int)__builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, 0);
-}
 // cache policy of the output stores: k_dslash's are non-temporal (2), so the
 // written lines, which this launch never reads again, do not displace the
 // neighbour gathers' source lines in L2 (FP32 CG iteration -0.8%, FP64 -1.8%
@@ -111,39 +84,6 @@ __device__ __forceinline__ void bstore(double2 v, Rsrc r, uint32_t voff, uint32_
 template <int POLICY>
 __device__ __forceinline__ void bstore(float2 v, Rsrc r, uint32_t voff, uint32_t soff) {
   __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(__attribute__((ext_vector_type(2))) unsigned, v), r, voff, soff, POLICY);
-}
-
-// A matrix operand: field descriptor, lane byte offset of the site, uniform
-// byte offset of element (0,0); element (i,j) is (i*NCOL+j) planes further.
-struct Opnd {
-  Rsrc r;
-  uint32_t v, s;
-};
-
-// acc += s * op(A) * op(B).  TA/TB select the dagger.  B is streamed one row
-// at a time (row j of op(B) meets column j of op(A)), so every operand
-// element is loaded once and only the accumulator plus one row stay live.
-template <typename R, bool TA, bool TB>
-__device__ __forceinline__ void mmacc(typename CT<R>::t (&acc)[NCOL][NCOL], R s, Opnd A,
-                                      Opnd B, uint32_t plane) {
-  typedef typename CT<R>::t C;
-#pragma unroll
-  for (int j = 0; j < NCOL; j++) {
-    C brow[NCOL];
-#pragma unroll
-    for (int k = 0; k < NCOL; k++) {
-      C v = bload<C>(B.r, B.v, B.s + (uint32_t)(TB ? k * NCOL + j : j * NCOL + k) * plane);
-      if (TB) v.y = -v.y;
-      brow[k] = v;
-    }
-#pragma unroll
-    for (int i = 0; i < NCOL; i++) {
-      C a = bload<C>(A.r, A.v, A.s + (uint32_t)(TA ? j * NCOL + i : i * NCOL + j) * plane);
-      R ar = s * a.x, ai = TA ? -s * a.y : s * a.y;
-#pragma unroll
-      for (int k = 0; k < NCOL; k++) cfma(acc[i][k], ar, ai, brow[k]);
-    }
-  }
 }
 
 template <typename R>
@@ -589,19 +529,8 @@ k_dslash_split(const typename CT<R>::t *__restrict__ src, typename CT<R>::t *__r
   const int L = blockIdx.x, lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int q = L >> 3, comp = q % NTF, qq = q / NTF;
-  int s;
-  bool live;
-  if (ord.paired) {
-    const int par = qq & 1, pos = qq >> 1;
-    const int chunk = (L & 7) * ord.slab + (ord.paired == 2 ? (pos % ord.T) * ord.P + pos / ord.T : pos);
-    const int i = chunk * 64 + lane;
-    s = par ? ord.half + i : i;
-    live = i < (par ? V - ord.half : ord.half);
-  } else {
-    s = ((L & 7) * ord.slab + qq) * 64 + lane;
-    live = s < V;
-  }
-  if (!live) s = 0;   // computes site 0 again and stores nothing
+  int s;   // (a lane without a site computes site 0 again and stores nothing)
+  const bool live = ord_site64(ord, L & 7, qq, lane, V, &s);
 
   const uint32_t cs = sizeof(C);
   const uint32_t pl = (uint32_t)V * cs;     // one element plane
@@ -861,7 +790,7 @@ static int dslash_launch(susy_ctx *c, const typename CT<R>::t *src,
                          const typename CT<R>::t *U, const typename CT<R>::t *Uinv,
                          const typename CT<R>::t *pdet, typename CT<R>::t *aux,
                          const int *skip, typename CT<R>::t *aux_out = nullptr,
-                         bool prep = true, bool sampled = true) {
+                         bool prep = true, bool sampled = true, bool keep_prep = false) {
   if (sign != 1 && sign != -1) {
     set_error("fermion_op: incorrect sign %d", sign);
     return SUSY_E_ARG;
@@ -873,7 +802,7 @@ static int dslash_launch(susy_ctx *c, const typename CT<R>::t *src,
   }
   if (sign != 1 || p0 != nullptr || !c->doG) aux_out = nullptr;
 #if NCOL <= 4
-  const bool split = ds_split<R>(V), inl = split && c->doG && prep && ds_split_inline(V);
+  const bool split = ds_split<R>(V), inl = split && c->doG && prep && !keep_prep && ds_split_inline(V);
 #else
   const bool split = false, inl = false;
 #endif
@@ -897,7 +826,8 @@ static int dslash_launch(susy_ctx *c, const typename CT<R>::t *src,
   const int threads = split ? 64 * DS_PARTS : DsSites<R>::n * DS_SPLIT * DsSites<R>::cpb;
   const int nb = ds_grid(V, c->p.nx * c->p.ny * c->p.nz,
                          sizeof(R) == sizeof(float) ? c->site_order32 : c->site_order,
-                         split ? 64 : DsSites<R>::n, &ord, split ? 1 : DsSites<R>::cpb);
+                         split ? 64 : DsSites<R>::n, &ord,
+                         split ? NTF : NTF / DsSites<R>::cpb);
   if (nblocks) *nblocks = nb;
   R pbc = (R)c->p.PBC, G = (R)c->p.G;
 #define DS_ARGS src, dst, U, Uinv, pdet, aux, aux_out, c->d_nbr, c->d_t, V, c->p.nt, pbc, \
@@ -983,6 +913,13 @@ int dslash64(susy_ctx *c, const double2 *src, double2 *dst, int sign,
              const double2 *p0, double shift, double *partial, int *nblocks, const int *skip) {
   return dslash_launch<double>(c, src, dst, sign, p0, shift, partial, nblocks,
                                c->d_links, c->d_uinv, c->d_pdet, c->d_aux, skip);
+}
+// dst = D src; with G terms also the traces Tr src_0, Tr(U_a^-1 src_{1+a}) in
+// d_aux and Tr(dst_0)^*, Tr(U_a^-1 dst_{1+a}^dag) in d_aux2 (6 planes each)
+int dslash64_traces(susy_ctx *c, const double2 *src, double2 *dst) {
+  return dslash_launch<double>(c, src, dst, 1, nullptr, 0.0, nullptr, nullptr, c->d_links,
+                               c->d_uinv, c->d_pdet, c->d_aux, nullptr, c->d_aux2, true, true,
+                               true);
 }
 int dslash32(susy_ctx *c, const float2 *src, float2 *dst, int sign,
              const float2 *p0, float shift, double *partial, int *nblocks, const int *skip) {

@@ -62,9 +62,10 @@
 struct DsOrder {
   int paired, slab, half, P, T;
 };
-// grid size (blocks) of the operator kernel, and its order parameters;
-// tslice = sites per t-slice (nx ny nz)
-inline int ds_grid(int V, int tslice, int paired, int DS_SITES, DsOrder *o, int cpb = 1) {
+// grid size (blocks) of a kernel with `parts` blocks per chunk (the operator:
+// its output components), and its order parameters; tslice = sites per t-slice
+// (nx ny nz)
+inline int ds_grid(int V, int tslice, int paired, int DS_SITES, DsOrder *o, int parts = NTF) {
   DsOrder d;
   d.paired = paired;
   d.half = V / 2;
@@ -83,12 +84,12 @@ inline int ds_grid(int V, int tslice, int paired, int DS_SITES, DsOrder *o, int 
       }
     }
     if (o) *o = d;
-    return 8 * d.slab * 2 * (NTF / cpb);
+    return 8 * d.slab * 2 * parts;
   }
   const int chunks = (V + DS_SITES - 1) / DS_SITES;
   d.slab = (chunks + 7) / 8;
   if (o) *o = d;
-  return 8 * d.slab * (NTF / cpb);
+  return 8 * d.slab * parts;
 }
 
 // ---------------------------------------------------------------------
@@ -241,7 +242,7 @@ struct susy_ctx {
   float2 *f_links = nullptr, *f_uinv = nullptr, *f_pdet = nullptr;
   int f_fresh = 0;                  // FP32 copies current?
   // operator scratch
-  double2 *d_aux = nullptr;         // 12 complex per site (operator/force prep)
+  double2 *d_aux = nullptr;         // 6 complex per site: operator prep
   float2 *f_aux = nullptr;
   double2 *d_aux2 = nullptr;        // 6 complex per site: D^dagger prep written by D
   float2 *f_aux2 = nullptr;
@@ -300,6 +301,7 @@ int dslash_init_tables(const PlaqTerms &pt);
 int dslash64(susy_ctx *c, const double2 *src, double2 *dst, int sign,
              const double2 *p0, double shift, double *partial, int *nblocks,
              const int *skip = nullptr);
+int dslash64_traces(susy_ctx *c, const double2 *src, double2 *dst);
 int dslash32(susy_ctx *c, const float2 *src, float2 *dst, int sign,
              const float2 *p0, float shift, double *partial, int *nblocks,
              const int *skip = nullptr);

@@ -111,3 +111,32 @@ def test_solver_scalar_steps(ncol, dims):
             r = src - lat.tf_download(h + 4) - shifts[j] * lat.tf_download(h + 1 + j)
             assert np.vdot(r, r).real <= margin * 1e-10 * n2, (form, j)
     lat.close()
+
+
+# The force's four waves a link share its terms by direction: sites below and
+# beyond a block, with and without the determinant terms, over two poles and
+# every site order.  Sums of some 70 products, relative to the whole force:
+# 1e-12 leaves three digits over their rounding.
+@pytest.mark.parametrize("ncol,dims", [(2, (2, 2, 2, 2)), (2, (6, 6, 6, 7)), (3, (1, 2, 3, 5)),
+                                       (3, (4, 5, 4, 6)), (4, (3, 3, 5, 2)), (4, (4, 4, 4, 10))])
+@pytest.mark.parametrize("G", [0.0, 0.2])
+def test_force_waves(ncol, dims, G):
+    print("force", ncol, dims, G, flush=True)
+    args = dict(dims=dims, iseed=5, kappa_u1=1.0, bmass=1.0, G=G)
+    O, lat = Oracle(ncol, **args), susy_amd.Lattice(ncol, **args)
+    lk = random_links(O.link_shape(), 3, 0.2)
+    O.set_links(lk)
+    lat.set_links(lk)
+    h = lat.tf_alloc(2)
+    sol = np.stack([random_tf(O.tf_shape(), 9), random_tf(O.tf_shape(), 10)])
+    for j in range(2):
+        lat.tf_upload(h + j, sol[j])
+    O.set_mom(np.zeros(O.link_shape(), complex))
+    O.fermion_force(0.1, sol, [0.7, -0.3])
+    want = O.get_mom()
+    for order in (0, 1, 2):
+        lat.set_site_order(order)
+        lat.set_mom(np.zeros(O.link_shape(), complex))
+        lat.fermion_force(0.1, h, [0.7, -0.3])
+        assert rel_err(lat.get_mom(), want) < 1e-12, order
+    lat.close()
