@@ -199,7 +199,7 @@ static int ctx_setup(susy_ctx *c) {
   const int tsl = p.nx * p.ny * p.nz;
   int ds_blocks = 0;
   for (int order = 0; order <= 2; order++)
-    for (int sites : {DS_SITES64, DS_SITES32, 64})
+    for (int sites : {256, 128, 64})
       ds_blocks = std::max(ds_blocks, ds_grid(V, tsl, order, sites, nullptr));
   c->npart = std::max({ds_blocks, 2048, 4 * ((V + 255) / 256), (NUMLINK * V + 255) / 256}) + 64;
   RET(dalloc(&c->d_part, (size_t)c->npart * 2));

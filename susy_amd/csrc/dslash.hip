@@ -176,10 +176,10 @@ k_dslash_prep_trace(const typename CT<R>::t *__restrict__ src,
 
 template <typename R> struct DsSites;
 template <> struct DsSites<double> {
-  static constexpr int n = DS_SITES64, waves = DS_WAVES64, cpb = DS_CPB64;
+  static constexpr int n = DS_SITES64, waves = DS_WAVES64;
 };
 template <> struct DsSites<float> {
-  static constexpr int n = DS_SITES32, waves = DS_WAVES32, cpb = DS_CPB32;
+  static constexpr int n = DS_SITES32, waves = DS_WAVES32;
 };
 
 // EPI = 0: dst = result.  EPI = 1: dst = result + shift * p0, and the block's
@@ -188,14 +188,10 @@ template <> struct DsSites<float> {
 // also store the pre-pass values of D^dagger applied to this output:
 // aux_out[0] = Tr(out_0)^*, aux_out[1+a] = Tr(U_a^-1 out_{1+a}^dag).
 //
-// A block covers DS_SITES sites of one output component.  With DS_SPLIT = 2
-// two threads share each output matrix: the first computes the site terms
-// a < 3, the first three Dminus terms, or Dplus and the first PtoP pair; the
-// second the rest and the G terms.  Their partial sums meet in LDS and the
-// first stores.  Fewer sites are then in flight per XCD at the same
-// occupancy, so their neighbourhoods compete less for the XCD's L2.
+// A block covers ord.sites sites (at most DsSites::n, see ds_sites) of one
+// output component.  (Two threads sharing an output matrix: 10-15% slower.)
 template <typename R, bool DAG, int EPI>
-__global__ void __launch_bounds__(DsSites<R>::n * DS_SPLIT * DsSites<R>::cpb)
+__global__ void __launch_bounds__(DsSites<R>::n)
     __attribute__((amdgpu_waves_per_eu(DsSites<R>::waves)))
 k_dslash(const typename CT<R>::t *__restrict__ src, typename CT<R>::t *__restrict__ dst,
          const typename CT<R>::t *__restrict__ U, const typename CT<R>::t *__restrict__ Uinv,
@@ -210,28 +206,21 @@ k_dslash(const typename CT<R>::t *__restrict__ src, typename CT<R>::t *__restric
   // (the flag is one word read by every thread: the exit is block-uniform)
   if (skip != nullptr && *skip) return;
   const int L = blockIdx.x;
-  constexpr int DS_SITES = DsSites<R>::n, CPB = DsSites<R>::cpb;
-  constexpr int DS_THREADS = DS_SITES * DS_SPLIT * CPB;
-  static_assert(CPB == 1 || DS_SPLIT == 1, "components per block need DS_SPLIT 1");
-  static_assert(NTF % CPB == 0 && DS_SITES % 64 == 0, "block shape");
-  const int lane = threadIdx.x % DS_SITES, w = CPB == 1 ? threadIdx.x / DS_SITES : 0;
-  const int q = L >> 3;                       // position in this XCD's queue
-  // a block holds CPB consecutive output components of one site chunk, one
-  // group of DS_SITES threads (whole wavefronts) per component
-  const int comp = CPB == 1 ? q % NTF : (q % (NTF / CPB)) * CPB + (int)threadIdx.x / DS_SITES;
-  const int qq = q / (NTF / CPB);             // chunk position in the queue
+  const int lane = threadIdx.x, sites = ord.sites;
+  const int q = L >> 3, comp = q % NTF;       // position in this XCD's queue
+  const int qq = q / NTF;                     // chunk position in the queue
   int s;
   bool live;
   if (ord.paired) {
     // even chunk k, odd chunk k, even chunk k+1, ... of this XCD's slab
     const int par = qq & 1, pos = qq >> 1;
     const int chunk = (L & 7) * ord.slab + (ord.paired == 2 ? (pos % ord.T) * ord.P + pos / ord.T : pos);
-    const int i = chunk * DS_SITES + lane;
+    const int i = chunk * sites + lane;
     s = par ? ord.half + i : i;
     live = i < (par ? V - ord.half : ord.half);
   } else {
     const int chunk = (L & 7) * ord.slab + qq;
-    s = chunk * DS_SITES + lane;
+    s = chunk * sites + lane;
     live = s < V;
   }
 
@@ -244,37 +233,48 @@ k_dslash(const typename CT<R>::t *__restrict__ src, typename CT<R>::t *__restric
   auto S = [&](int k, int x) { return Opnd{rS, (uint32_t)x * cs, (uint32_t)k * Mb}; };
   auto Ul = [&](int a, int x) { return Opnd{rU, (uint32_t)x * cs, (uint32_t)a * Mb}; };
 
+  // The determinant sums' gathered scalars: 20 (site) or 4 (link) round trips
+  // to memory one after the other were up to a third of a wave's time, so
+  // their loads go out together.  FP64 from U(4) on is bound by what the L2
+  // misses, and loses by it.  us of a CG iteration, in turn | together: U(4)
+  // FP32 8^3x16 107 | 99, 12^3x24 462 | 453, 16^4 738 | 730; U(3) FP64 8^3x16 89.3
+  // | 86.5, 16^4 712 | 706; but U(4) FP64 16^4 1337 | 1394.
+  constexpr bool det_together = sizeof(R) == 4 || NCOL <= 3;
+  constexpr int det_unroll = det_together ? NUMLINK : 1;
   C acc[NCOL][NCOL];
 #pragma unroll
   for (int i = 0; i < NCOL; i++)
 #pragma unroll
     for (int k = 0; k < NCOL; k++) acc[i][k] = mkc<C>(0, 0);
-  const bool first = DS_SPLIT == 1 || w == 0, last = DS_SPLIT == 1 || w == DS_SPLIT - 1;
 
   if (live) {
     const int t = tco[s];
 
     if (comp == 0) {
       // ---- site output: 1/2 sum_a [psi_a(x) Ubar_a(x) - bc(-a) Ubar_a(x-a) psi_a(x-a)]
-      const int a0 = first ? 0 : 3, a1 = last ? NUMLINK : 3;
       DS_UNROLL_LOOP(DS_UNROLL)
-      for (int a = a0; a < a1; a++) {
+      for (int a = 0; a < NUMLINK; a++) {
         const int xm = nb(g_bwd(a));
         mmacc<R, DAG, true>(acc, (R)0.5, S(1 + a, s), Ul(a, s), pl);
         mmacc<R, true, DAG>(acc, (R)-0.5 * bcsign<R>(t, -link_tau(a), nt, pbc), Ul(a, xm),
                             S(1 + a, xm), pl);
       }
-      if (doG && last) {
+      if (doG) {
         // detLtoS: -(i G C2 sqrt(N)/2) sum_{a!=b} plaqdet_ab [T_b(x) + bc(b) T_a(x+b)]
         //          * Lambda_{DIMF-1},  Lambda_{DIMF-1} = i I / sqrt(N)
         const Rsrc rA = make_rsrc(aux, 6 * pl), rP = make_rsrc(pdet, NUMLINK * NUMLINK * pl);
         C sum = mkc<C>(0, 0);
-#pragma unroll 1
+        int xf[NUMLINK];
+#pragma unroll
+        for (int b = 0; b < NUMLINK; b++)
+          if (det_together) xf[b] = nb(g_fwd(b));
+        DS_UNROLL_LOOP(det_unroll)
         for (int b = 0; b < NUMLINK; b++) {
-          const int xb = nb(g_fwd(b));
+          if (det_together && sizeof(R) == 8) __builtin_amdgcn_sched_barrier(0);
+          const int xb = det_together ? xf[b] : nb(g_fwd(b));
           const C tb = bload<C>(rA, (uint32_t)s * cs, (1 + b) * pl);
           const R sg = bcsign<R>(t, link_tau(b), nt, pbc);
-#pragma unroll 1
+          DS_UNROLL_LOOP(det_unroll)
           for (int a = 0; a < NUMLINK; a++) {
             if (a == b) continue;
             const C ta = bload<C>(rA, (uint32_t)xb * cs, (1 + a) * pl);
@@ -299,8 +299,6 @@ k_dslash(const typename CT<R>::t *__restrict__ src, typename CT<R>::t *__restric
       DS_UNROLL_LOOP(DS_UNROLL)
       for (int a = 0; a < NUMLINK; a++) {
         if (a == b) continue;
-        // the first thread takes the first three a != b, the other the last
-        if (DS_SPLIT == 2 && ((a - (a > b)) < 3) != first) continue;
         // Dminus: U_a(x+b) chi_ab(x) - bc(-a) chi_ab(x-a) U_a(x-a)
         const int xm = nb(g_bwd(a));
         const R sg = a < b ? (R)1 : (R)-1;   // chi_ab = sg * stored chi_{min,max}
@@ -309,21 +307,20 @@ k_dslash(const typename CT<R>::t *__restrict__ src, typename CT<R>::t *__restric
         mmacc<R, DAG, false>(acc, -sg * bcsign<R>(t, -link_tau(a), nt, pbc), S(pc, xm),
                              Ul(a, xm), pl);
       }
-      if (last) {
-        // DbplusStoL: 1/2 [bc(b) eta(x+b) Ubar_b(x) - Ubar_b(x) eta(x)]
-        mmacc<R, DAG, true>(acc, (R)0.5 * bcsign<R>(t, link_tau(b), nt, pbc), S(0, xb),
-                            Ul(b, s), pl);
-        mmacc<R, true, DAG>(acc, (R)-0.5, Ul(b, s), S(0, s), pl);
-      }
-      if (doG && last) {
+      // DbplusStoL: 1/2 [bc(b) eta(x+b) Ubar_b(x) - Ubar_b(x) eta(x)]
+      mmacc<R, DAG, true>(acc, (R)0.5 * bcsign<R>(t, link_tau(b), nt, pbc), S(0, xb), Ul(b, s),
+                          pl);
+      mmacc<R, true, DAG>(acc, (R)-0.5, Ul(b, s), S(0, s), pl);
+      if (doG) {
         // detStoL: -G C2/2 U_b^-1(x) sum_{c!=b} [Tr eta(x) plaqdet_cb(x)
         //                                        + bc(-c) Tr eta(x-c) plaqdet_bc(x-c)]
         const Rsrc rA = make_rsrc(aux, 6 * pl), rP = make_rsrc(pdet, NUMLINK * NUMLINK * pl);
         const Rsrc rI = make_rsrc(Uinv, NUMLINK * Mb);
         C sum = mkc<C>(0, 0);
         const C te = bload<C>(rA, (uint32_t)s * cs, 0);
-#pragma unroll 1
-        for (int c = 0; c < NUMLINK; c++) {
+        DS_UNROLL_LOOP(det_unroll)
+        for (int n = 0; n < (det_together ? NUMLINK - 1 : NUMLINK); n++) {
+          const int c = det_together ? n + (n >= b) : n;
           if (c == b) continue;
           const int xm = nb(g_bwd(c));
           const C p1 = bload<C>(rP, (uint32_t)s * cs, (c * NUMLINK + b) * pl);
@@ -351,15 +348,10 @@ k_dslash(const typename CT<R>::t *__restrict__ src, typename CT<R>::t *__restric
       const int xa = nb(g_fwd(a)), xb = nb(g_fwd(b));
       // Dplus: bc(a) U_a(x) psi_b(x+a) - psi_b(x) U_a(x+b)
       //        - bc(b) U_b(x) psi_a(x+b) + psi_a(x) U_b(x+a)
-      if (first) {
-        mmacc<R, false, DAG>(acc, bcsign<R>(t, link_tau(a), nt, pbc), Ul(a, s), S(1 + b, xa),
-                             pl);
-        mmacc<R, DAG, false>(acc, (R)-1, S(1 + b, s), Ul(a, xb), pl);
-        mmacc<R, false, DAG>(acc, -bcsign<R>(t, link_tau(b), nt, pbc), Ul(b, s), S(1 + a, xb),
-                             pl);
-        mmacc<R, DAG, false>(acc, (R)1, S(1 + a, s), Ul(b, xa), pl);
-      }
-      const int n0 = first ? 0 : 1, n1 = last ? 3 : 1;
+      mmacc<R, false, DAG>(acc, bcsign<R>(t, link_tau(a), nt, pbc), Ul(a, s), S(1 + b, xa), pl);
+      mmacc<R, DAG, false>(acc, (R)-1, S(1 + b, s), Ul(a, xb), pl);
+      mmacc<R, false, DAG>(acc, -bcsign<R>(t, link_tau(b), nt, pbc), Ul(b, s), S(1 + a, xb), pl);
+      mmacc<R, DAG, false>(acc, (R)1, S(1 + a, s), Ul(b, xa), pl);
       // DbplusPtoP + DbminusPtoP.  Each DbminusPtoP term landing on (a,b)
       // coincides with the DbplusPtoP term of the same c: with (d,e) the
       // other two links, x-d-e = x+a+b+c and x-d-e-c = x+a+b (the five e_a
@@ -367,7 +359,7 @@ k_dslash(const typename CT<R>::t *__restrict__ src, typename CT<R>::t *__restric
       // offsets agree for the same reason.  The DbplusPtoP terms are applied
       // at double weight (checked term by term when the tables are built).
       DS_UNROLL_LOOP(DS_UNROLL)
-      for (int n = n0; n < n1; n++) {
+      for (int n = 0; n < 3; n++) {
         const int c = c_pt.pp_c[p][n];
         const int pc = 6 + c_pt.pp_de[p][n];
         const int x1 = nb(c_pt.pp_g1[p][n]), x2 = nb(c_pt.pp_g2[p][n]), xmc = nb(g_bwd(c));
@@ -380,32 +372,8 @@ k_dslash(const typename CT<R>::t *__restrict__ src, typename CT<R>::t *__restric
     }
   }
 
-#if DS_SPLIT > 1
-  // the second thread's partial sum meets the first's in LDS
-  __shared__ C part[DS_SPLIT - 1][NN][DS_SITES];
-  if (!first) {
-#pragma unroll
-    for (int i = 0; i < NCOL; i++)
-#pragma unroll
-      for (int k = 0; k < NCOL; k++) part[w - 1][i * NCOL + k][lane] = acc[i][k];
-  }
-  __syncthreads();
-  if (first) {
-#pragma unroll
-    for (int u = 0; u < DS_SPLIT - 1; u++)
-#pragma unroll
-      for (int i = 0; i < NCOL; i++)
-#pragma unroll
-        for (int k = 0; k < NCOL; k++) {
-          const C v = part[u][i * NCOL + k][lane];
-          acc[i][k].x += v.x;
-          acc[i][k].y += v.y;
-        }
-  }
-#endif
-
   double dot = 0.0;
-  if (live && first) {
+  if (live) {
     // ---- epilogue loads (p0 for the DSq epilogue, U^-1 for the D^dagger
     // pre-pass values), all drained before the first store
     const Rsrc rD = make_rsrc(dst, NTF * Mb);
@@ -472,12 +440,12 @@ k_dslash(const typename CT<R>::t *__restrict__ src, typename CT<R>::t *__restric
   if (EPI == 1) {
     // deterministic block reduction: wavefront butterfly, then across waves
     for (int off = 32; off > 0; off >>= 1) dot += __shfl_xor(dot, off, 64);
-    __shared__ double red[DS_THREADS / 64];
+    __shared__ double red[DsSites<R>::n / 64];
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = dot;
     __syncthreads();
     if (threadIdx.x == 0) {
       double tsum = 0;
-      for (int u = 0; u < DS_THREADS / 64; u++) tsum += red[u];
+      for (int u = 0; u < sites / 64; u++) tsum += red[u];
       partial[L] = tsum;
     }
   }
@@ -763,17 +731,19 @@ k_dslash_split(const typename CT<R>::t *__restrict__ src, typename CT<R>::t *__r
 // k_dslash wins where a launch fills the chip.  Both sides, us of a CG
 // iteration, which leaves less of the operands in the caches than an operator
 // that is repeated alone, k_dslash | k_dslash_split:
-//   U(4) FP64  1296: 87.0 | 62.2    2160: 93.0 | 78.5    4096: 105.9 | 103.0
-//              8192: 168.9 | 183.6  (4096 sites alone: D 27.3 | 29.6)
-//        FP32  2160: 78.4 | 61.5    4096: 83.1 | 76.5    8192: 117.2 | 122.9
-//   U(3) FP64  1296: 61.5 | 48.0    2160: 64.2 | 57.5    4096: 68.2 | 71.9
-//        FP32  8192: 80.2 | 75.5   20736: 162.2 | 149.8 65536: 420.3 | 423.2
-//   U(2) FP64  8192: 62.8 | 61.9   20736: 136.8 | 116.6 65536: 320.7 | 328.2
-//        FP32  8192: 56.3 | 52.8   20736: 96.7 | 86.9   65536: 208.5 | 210.2
+//   U(4) FP64  2160: 74.3 | 64.4    4096: 92.5 | 88.6    8192: 154 | 165
+//        FP32  1296: 48.5 | 39.7    2160: 54.7 | 49.4    4096: 61.6 | 63.1
+//   U(3) FP64  2160: 46.2 | 44.9    4096: 54.3 | 58.4    8192: 86.7 | 102.8
+//        FP32  8192: 62.6 | 63.3   16384: 110 | 107     20736: 142 | 134
+//             65536: 404 | 418
+//   U(2) FP64  4096: 31.1 | 31.4    8192: 47.2 | 49.0   20736: 109 | 101
+//             32768: 153 | 147     65536: 294 | 322
+//        FP32  8192: 41.6 | 42.7   20736: 82.4 | 76.5   32768: 110 | 108
+//             65536: 191 | 192
 template <typename R>
 static bool ds_split(int V) {
   const bool dbl = sizeof(R) == sizeof(double);
-  return V <= (NCOL == 2 || (NCOL == 3 && !dbl) ? 32768 : dbl ? 3072 : 6144);
+  return V <= (NCOL == 2 || (NCOL == 3 && !dbl) ? 32768 : NCOL == 4 && dbl ? 4096 : 3072);
 }
 
 // Where it also makes the pre-pass values itself: the launch of k_dslash_prep
@@ -823,11 +793,11 @@ static int dslash_launch(susy_ctx *c, const typename CT<R>::t *src,
     HIPCHK(hipGetLastError());
   }
   DsOrder ord;
-  const int threads = split ? 64 * DS_PARTS : DsSites<R>::n * DS_SPLIT * DsSites<R>::cpb;
+  const int sites = split ? 64 : ds_sites(V, DsSites<R>::n);
+  const int threads = split ? 64 * DS_PARTS : sites;
   const int nb = ds_grid(V, c->p.nx * c->p.ny * c->p.nz,
                          sizeof(R) == sizeof(float) ? c->site_order32 : c->site_order,
-                         split ? 64 : DsSites<R>::n, &ord,
-                         split ? NTF : NTF / DsSites<R>::cpb);
+                         sites, &ord);
   if (nblocks) *nblocks = nb;
   R pbc = (R)c->p.PBC, G = (R)c->p.G;
 #define DS_ARGS src, dst, U, Uinv, pdet, aux, aux_out, c->d_nbr, c->d_t, V, c->p.nt, pbc, \

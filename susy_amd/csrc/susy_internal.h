@@ -26,25 +26,13 @@
 #define NTERMS 30
 #define NQLINK 28
 #define IMAG_TOL 1.0e-8
-// operator kernel: a block covers DS_SITES64 (FP64) / DS_SITES32 (FP32)
-// sites of one output component, with DS_SPLIT wavefronts sharing the
-// products of each output matrix (measured best: 256 / 128 / 1)
+// operator kernel: a block covers up to DS_SITES64 (FP64) / DS_SITES32 (FP32)
+// sites of one output component (measured best: 256 / 128)
 #ifndef DS_SITES64
 #define DS_SITES64 256
 #endif
 #ifndef DS_SITES32
 #define DS_SITES32 128
-#endif
-#ifndef DS_SPLIT
-#define DS_SPLIT 1
-#endif
-// output components per block of the operator kernel (each a whole number
-// of wavefronts over the block's site chunk); 1 = one component per block
-#ifndef DS_CPB64
-#define DS_CPB64 1
-#endif
-#ifndef DS_CPB32
-#define DS_CPB32 1
 #endif
 #define C2 1.0
 
@@ -61,6 +49,7 @@
 //     slab to hold whole t-slices of whole chunks; otherwise it is order 1.
 struct DsOrder {
   int paired, slab, half, P, T;
+  int sites;   // of a chunk
 };
 // grid size (blocks) of a kernel with `parts` blocks per chunk (the operator:
 // its output components), and its order parameters; tslice = sites per t-slice
@@ -70,6 +59,7 @@ inline int ds_grid(int V, int tslice, int paired, int DS_SITES, DsOrder *o, int 
   d.paired = paired;
   d.half = V / 2;
   d.P = d.T = 1;
+  d.sites = DS_SITES;
   if (paired) {
     const int chunks = (V - d.half + DS_SITES - 1) / DS_SITES;   // odd half is the larger
     d.slab = (chunks + 7) / 8;
@@ -90,6 +80,18 @@ inline int ds_grid(int V, int tslice, int paired, int DS_SITES, DsOrder *o, int 
   d.slab = (chunks + 7) / 8;
   if (o) *o = d;
   return 8 * d.slab * parts;
+}
+
+// Sites of the operator kernel's blocks: the largest of most, 128 and 64 whose
+// chunks the 8 XCDs can share to 2%, since the XCD with one more chunk is
+// waited for: a half of 12^3x24 is 81 chunks of 256, 11 on one XCD for a mean
+// of 10.1 (FP64 CG iteration at U(4) 915 -> 876 us with 64 sites, U(3) 12^4 251
+// -> 235); equal shares are a little faster in large chunks (16^4 1337 | 1350).
+inline int ds_sites(int V, int most) {
+  auto share = [&](int n) { return ((V - V / 2 + n - 1) / n + 7) / 8 * n; };
+  int n = most;
+  while (n > 64 && share(n) * 50L > share(64) * 51L) n /= 2;
+  return n;
 }
 
 // ---------------------------------------------------------------------

@@ -18,7 +18,8 @@ def pair(ncol, dims, **kw):
 # The smallest lattices, halves that are no multiple of the 64 sites of a
 # block, odd extents (no even-odd halves of one size), and both sides of the
 # limits: U(2) pre-pass in the kernel up to 1296 sites, five waves up to 32768
-# (U(2), and U(3) FP32), 3072 (FP64) and 6144 (U(4) FP32).
+# (U(2), and U(3) FP32), 4096 (U(4) FP64) and 3072 (U(3) FP64, U(4) FP32); above,
+# blocks of 64, 128 and 256 sites, by what divides the lattice among 8 XCDs.
 # Bounds: a result sums some 20 NCOL products of order one, so rounding is
 # about 1e-15 (FP64) and 6e-7 (FP32) of the largest element.
 @pytest.mark.parametrize("ncol,dims", [
@@ -27,7 +28,7 @@ def pair(ncol, dims, **kw):
     (3, (1, 2, 3, 5)), (3, (8, 8, 8, 6)), (3, (8, 8, 7, 7)), (3, (16, 16, 16, 8)),
     (3, (16, 15, 18, 8)),
     (4, (2, 2, 2, 2)), (4, (3, 3, 5, 2)), (4, (8, 8, 8, 6)), (4, (8, 8, 7, 7)),
-    (4, (8, 8, 12, 8)), (4, (8, 8, 7, 14)),
+    (4, (8, 8, 8, 8)), (4, (8, 8, 7, 10)), (4, (8, 8, 12, 8)), (4, (8, 8, 7, 14)),
 ])
 def test_operator_across_limits(ncol, dims):
     print("operator", ncol, dims, flush=True)
