@@ -236,10 +236,12 @@ k_dslash(const typename CT<R>::t *__restrict__ src, typename CT<R>::t *__restric
   // The determinant sums' gathered scalars: 20 (site) or 4 (link) round trips
   // to memory one after the other were up to a third of a wave's time, so
   // their loads go out together.  FP64 from U(4) on is bound by what the L2
-  // misses, and loses by it.  us of a CG iteration, in turn | together: U(4)
-  // FP32 8^3x16 107 | 99, 12^3x24 462 | 453, 16^4 738 | 730; U(3) FP64 8^3x16 89.3
-  // | 86.5, 16^4 712 | 706; but U(4) FP64 16^4 1337 | 1394.
-  constexpr bool det_together = sizeof(R) == 4 || NCOL <= 3;
+  // misses, and loses by it; so does FP32 at U(5), at every size (with the same
+  // three waves per SIMD).  us of a CG iteration, in turn | together: U(4) FP32
+  // 8^3x16 107 | 99, 12^3x24 462 | 453, 16^4 738 | 730; U(3) FP64 8^3x16 89.3 |
+  // 86.5, 16^4 712 | 706; but U(4) FP64 16^4 1337 | 1394, U(5) FP32 4^4 75 | 92,
+  // 8^4 125 | 161, 8^3x16 176 | 211, 12^4 438 | 495, 16^4 1333 | 1438.
+  constexpr bool det_together = NCOL <= 3 || (sizeof(R) == 4 && NCOL == 4);
   constexpr int det_unroll = det_together ? NUMLINK : 1;
   C acc[NCOL][NCOL];
 #pragma unroll

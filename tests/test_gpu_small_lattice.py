@@ -141,3 +141,19 @@ def test_force_waves(ncol, dims, G):
         lat.fermion_force(0.1, h, [0.7, -0.3])
         assert rel_err(lat.get_mom(), want) < 1e-12, order
     lat.close()
+
+
+# U(5): the operator's ordinary kernel takes its determinant scalars one after
+# the other in both precisions, and the force's waves make two columns each,
+# in rounds of three and two rows.  Site counts below one block, beyond it
+# with a remainder in each half, and over several XCDs; inputs and bounds are
+# those of the tests above.
+@pytest.mark.parametrize("dims", [(3, 3, 5, 2), (4, 4, 5, 2), (4, 6, 5, 6)])
+def test_operator_u5_blocks(dims):
+    test_operator_across_limits(5, dims)
+
+
+@pytest.mark.parametrize("dims", [(3, 3, 5, 2), (4, 4, 5, 2), (4, 6, 5, 6)])
+@pytest.mark.parametrize("G", [0.0, 0.2])
+def test_force_u5_blocks(dims, G):
+    test_force_waves(5, dims, G)
