@@ -561,13 +561,22 @@ extern "C" int susy_set_cg_options(int window, int reliable) {
 // them itself and one block beside them advances the scalar state: an
 // iteration is then four launches, where k_cgs_beta and k_cgs_alpha make it
 // six (and a launch per reduction, recurrence and stopping test made it nine).
-// Above, the blocks' sums cost more than the two launches.  us of an
-// iteration, nine | six | four launches:
+// Above, the blocks' sums cost more than the two launches; FP64 hides more of
+// them behind its fields.  us of an iteration, nine | six | four launches:
 //   U(2) 4^4 FP64 31.1 | 26.4 | 22.1       U(3) 4^4 FP32 32.2 | 27.5 | 22.3
 //   U(4) 4^3x8 FP32 38.8 | 32.8 | 28.7     U(4) 8^3x16 FP32 117.1 | 110.2 | 107.3
-//   U(2) 8^2x16^2 FP64 91.7 | 83.8 | 81.0  U(2) 16^4 FP32 201.8 | 199.4 | 202.2
-//   U(2) 16^3x32 FP32 (32768 partials) 394 | 386 | 396
-#define CG_SUM_PARTS 8192
+// and six | four where the limits lie, with the number of partials:
+//   FP32  5376: U(2) 12^4 77.4 | 77.1, U(3) 12^4 136.0 | 134.6
+//         6144: U(2) 16^3x6 86.3 | 86.5, U(3) 16^3x6 154.1 | 152.2,
+//               U(4) 16^3x12 548.2 | 547.0, U(3) 16^3x12 300.9 | 302.2
+//         6912: U(2) 12^3x16 93.0 | 94.9, U(3) 169.2 | 168.8, U(4) 302.8 | 305.1
+//         8192: U(2) 16^4 195.7 | 199.0, U(3) 16^4 416.9 | 420.9
+//   FP64  6912: U(2) 12^3x16 130.8 | 127.9, U(3) 306.3 | 306.8
+//         8192: U(2) 16^3x8 152.2 | 148.7, 16^3x32 650.8 | 648.2,
+//               U(4) 16^3x32 2850 | 2857 (0.2% given away)
+//        10496: U(2) 12^3x24 198.4 | 198.7, U(3) 464.5 | 464.2
+template <typename C>
+constexpr int cg_sum_parts = sizeof(C) == sizeof(double2) ? 8192 : 6144;
 
 // iterations enqueued between two read-backs of the solver status
 #define CG_BATCH 16
@@ -724,7 +733,7 @@ static int cg_impl(susy_ctx *c, const double2 *src, double2 *const *psim, int ns
       for (int k = 0; k < CG_BATCH; k++) {
         int nbd;
         if ((e = dsq(pcur, ap, &nbd, p_prepped))) return e;
-        const bool sum = nbd <= CG_SUM_PARTS;
+        const bool sum = nbd <= cg_sum_parts<C>;
         C *rnew = slot(host_cnt);
         C *pnext = pcur != pfrozen ? pcur : (pcur == p0buf[0] ? p0buf[1] : p0buf[0]);
         const unsigned nbp = (c->V + CB - 1) / CB;

@@ -80,8 +80,8 @@ def test_surrogate_site_blocks(ncol, dims):
     lat.close()
 
 
-# The two ways of an iteration's scalar steps: blocks that sum up to 8192
-# partials themselves (the last size of it) and one block above.  The first 12
+# The iteration's scalar steps, from few partials up to 8192, the last number
+# that the blocks of FP64 sum themselves (test_solver_routes: both sides).  The first 12
 # iterations follow the oracle to rounding (later ones amplify it: on the U(3)
 # lattice |r|^2 of any two roundings differs by 1e-5 after 40 and by a tenth
 # after 46); at the end every system's true residual is below the bound, with
@@ -157,3 +157,50 @@ def test_operator_u5_blocks(dims):
 @pytest.mark.parametrize("G", [0.0, 0.2])
 def test_force_u5_blocks(dims, G):
     test_force_waves(5, dims, G)
+
+
+def partials(dims, chunk):
+    """blocks of the operator, one partial of <p, A p> each, in chunks of
+    `chunk` sites of both halves of the site order, shared by 8 XCDs"""
+    vol = int(np.prod(dims))
+    chunks = -(-(vol - vol // 2) // chunk)
+    return 8 * -(-chunks // 8) * 2 * 16
+
+
+# The two ways of an iteration's scalar steps at their limits, 8192 partials in
+# FP64 and 6144 in FP32: every block sums them (four launches) or one block does
+# (six).  All these lattices work in chunks of 64 sites.  Both forms follow the
+# oracle's first 12 iterations: FP64 as in test_solver_scalar_steps; in FP32 every
+# iteration adds its roundings of some 6e-7 to vectors that the shifted operator
+# (condition below 1e3 on these links) amplifies by less than 100 in all.  At
+# the end the true residuals are below the bound, with that test's margins.
+@pytest.mark.parametrize("dims,four64,four32", [((16, 16, 16, 6), True, True),
+                                                ((12, 12, 12, 16), True, False),
+                                                ((12, 12, 12, 24), False, False)])
+def test_solver_routes(dims, four64, four32):
+    print("solver routes", dims, flush=True)
+    n = partials(dims, 64)
+    assert (n <= 8192, n <= 6144) == (four64, four32)
+    O, lat = pair(2, dims)
+    lk = random_links(O.link_shape(), 3, 0.2)
+    O.set_links(lk)
+    lat.set_links(lk)
+    src = random_tf(O.tf_shape(), 9)
+    shifts = [0.5, 2.0, 9.0]
+    h = lat.tf_alloc(5)
+    lat.tf_upload(h, src)
+    it_o, sz_o, psi = O.congrad_multi(src, shifts, 12, 1e-10)
+    n2 = np.vdot(src, src).real
+    for form, sz_tol, tol, margin in ((susy_amd.FORM_FP64, 1e-6, 1e-10, 1.01),
+                                      (susy_amd.FORM_FP32, 1e-3, 1e-4, 4)):
+        it, sz = lat.congrad_multi(h, h + 1, shifts, 12, 1e-10, form)
+        assert it == it_o == 12
+        assert abs(sz / sz_o - 1) < sz_tol, form
+        for j in range(3):
+            assert rel_err(lat.tf_download(h + 1 + j), psi[j]) < tol, (form, j)
+        assert lat.congrad_multi(h, h + 1, shifts, 500, 1e-10, form)[0] < 500
+        for j in range(3):
+            lat.dsq(h + 1 + j, h + 4)
+            r = src - lat.tf_download(h + 4) - shifts[j] * lat.tf_download(h + 1 + j)
+            assert np.vdot(r, r).real <= margin * 1e-10 * n2, (form, j)
+    lat.close()
