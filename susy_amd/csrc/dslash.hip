@@ -733,25 +733,33 @@ k_dslash_split(const typename CT<R>::t *__restrict__ src, typename CT<R>::t *__r
 // k_dslash wins where a launch fills the chip.  Both sides, us of a CG
 // iteration, which leaves less of the operands in the caches than an operator
 // that is repeated alone, k_dslash | k_dslash_split:
-//   U(4) FP64  2160: 74.3 | 64.4    4096: 92.5 | 88.6    8192: 154 | 165
-//        FP32  1296: 48.5 | 39.7    2160: 54.7 | 49.4    4096: 61.6 | 63.1
-//   U(3) FP64  2160: 46.2 | 44.9    4096: 54.3 | 58.4    8192: 86.7 | 102.8
-//        FP32  8192: 62.6 | 63.3   16384: 110 | 107     20736: 142 | 134
-//             65536: 404 | 418
-//   U(2) FP64  4096: 31.1 | 31.4    8192: 47.2 | 49.0   20736: 109 | 101
-//             32768: 153 | 147     65536: 294 | 322
-//        FP32  8192: 41.6 | 42.7   20736: 82.4 | 76.5   32768: 110 | 108
-//             65536: 191 | 192
+//   U(4) FP64  2160: 74.5 | 64.3    4096: 92.1 | 88.0    8192: 154 | 165
+//        FP32  2160: 55.7 | 49.4    3072: 56.8 | 50.8    4096: 63.6 | 64.1
+//   U(3) FP64  2160: 46.5 | 44.7    3072: 49.6 | 47.4    4096: 55.1 | 58.6
+//        FP32  4096: 43.3 | 40.6    8192: 63.8 | 63.1   16384: 111 | 108
+//             32768: 209 | 199     49152: 303 | 299     65536: 404 | 418
+//   U(2) FP64  4096: 32.0 | 31.5    6144: 40.9 | 40.0    8192: 48.3 | 49.1
+//              9216: 54.2 | 52.6   16384: 82.8 | 80.6   32768: 156 | 148
+//             49152: 229 | 231     65536: 294 | 322
+//        FP32  2048: 26.0 | 24.2    3072: 28.3 | 27.5    3584: 29.9 | 30.6
+//              4096: 29.3 | 31.0    5120: 33.5 | 34.5    6144: 35.2 | 35.9
+//              6912: 39.1 | 38.3    8192: 41.5 | 42.3    9216: 45.4 | 44.6
+//             16384: 64.7 | 64.1   32768: 111 | 110     65536: 191 | 192
+// U(2) FP32 gives the sizes between 3072 and 6144 back to k_dslash; 2% at 6144
+// and 8192 (and at 8192 in FP64) are left to this kernel, which is the faster
+// one at 6912 and from 9216 on, and alone at 6144 (10.7 us of 11.2).
 template <typename R>
 static bool ds_split(int V) {
   const bool dbl = sizeof(R) == sizeof(double);
+  if (NCOL == 2 && !dbl && V > 3072 && V < 6144) return false;
   return V <= (NCOL == 2 || (NCOL == 3 && !dbl) ? 32768 : NCOL == 4 && dbl ? 4096 : 3072);
 }
 
-// Where it also makes the pre-pass values itself: the launch of k_dslash_prep
-// is 1.6 us of 6.3 on U(2) 4^4 and still wins a little at 6^4 (7.7 -> 7.5);
-// with the larger matrices the ten more products cost more than it (U(3) 4^4
-// 7.9 -> 10.0, U(4) 4^3x8 10.2 -> 12.3).
+// Where it also makes the pre-pass values itself instead of a launch of their
+// own (us of an operator, launch | inside, FP64, FP32): U(2) 256 sites 6.3 | 4.7,
+// 6.1 | 4.8; 1296 7.8 | 7.6, 7.3 | 7.1; 2160 9.0 | 8.1, 8.1 | 9.3; 4096 10.3 | 10.7,
+// 9.1 | 11.1.  With the larger matrices the ten more products cost more than
+// the launch (U(3) 4^4 7.9 | 10.0, U(4) 4^3x8 10.2 | 12.3).
 static constexpr bool ds_split_inline(int V) { return NCOL == 2 && V <= 1296; }
 #endif  // NCOL <= 4
 

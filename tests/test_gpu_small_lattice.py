@@ -204,3 +204,13 @@ def test_solver_routes(dims, four64, four32):
             r = src - lat.tf_download(h + 4) - shifts[j] * lat.tf_download(h + 1 + j)
             assert np.vdot(r, r).real <= margin * 1e-10 * n2, (form, j)
     lat.close()
+
+
+# Limits that test_operator_across_limits does not reach: U(2) in FP32 takes
+# the ordinary kernel between 3072 and 6144 sites, the five waves on both sides of
+# that range; the pre-pass has a thread per site and trace up to 65536 sites
+# and a thread per site above.
+@pytest.mark.parametrize("dims", [(8, 8, 8, 6), (8, 8, 7, 7), (8, 8, 10, 8), (8, 8, 8, 12),
+                                  (16, 16, 16, 16), (16, 16, 16, 17)])
+def test_operator_more_limits(dims):
+    test_operator_across_limits(2, dims)
