@@ -64,21 +64,26 @@ __device__ __forceinline__ void mmacc(typename CT<R>::t (&acc)[NCOL][NCOL], R s,
   }
 }
 
-// Site of a lane in the block order `ord` with chunks of 64 sites: qq is the
-// chunk's position in the queue of XCD x.  False: no such site (0 is given).
-__device__ __forceinline__ bool ord_site64(const DsOrder &ord, int x, int qq, int lane, int V,
-                                           int *s) {
-  bool live;
+// Site of a lane in the block order `ord` with chunks of `sites` sites: qq is
+// the chunk's position in the queue of XCD x.  False: no such site (*s is then
+// out of range).
+__device__ __forceinline__ bool ord_site(const DsOrder &ord, int sites, int x, int qq, int lane,
+                                         int V, int *s) {
   if (ord.paired) {
+    // even chunk k, odd chunk k, even chunk k+1, ... of this XCD's slab
     const int par = qq & 1, pos = qq >> 1;
     const int chunk = x * ord.slab + (ord.paired == 2 ? (pos % ord.T) * ord.P + pos / ord.T : pos);
-    const int i = chunk * 64 + lane;
+    const int i = chunk * sites + lane;
     *s = par ? ord.half + i : i;
-    live = i < (par ? V - ord.half : ord.half);
-  } else {
-    *s = (x * ord.slab + qq) * 64 + lane;
-    live = *s < V;
+    return i < (par ? V - ord.half : ord.half);
   }
+  *s = (x * ord.slab + qq) * sites + lane;
+  return *s < V;
+}
+// The same for chunks of 64 sites, with site 0 given to a lane that has none.
+__device__ __forceinline__ bool ord_site64(const DsOrder &ord, int x, int qq, int lane, int V,
+                                           int *s) {
+  const bool live = ord_site(ord, 64, x, qq, lane, V, s);
   if (!live) *s = 0;
   return live;
 }

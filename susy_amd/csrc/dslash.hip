@@ -210,19 +210,7 @@ k_dslash(const typename CT<R>::t *__restrict__ src, typename CT<R>::t *__restric
   const int q = L >> 3, comp = q % NTF;       // position in this XCD's queue
   const int qq = q / NTF;                     // chunk position in the queue
   int s;
-  bool live;
-  if (ord.paired) {
-    // even chunk k, odd chunk k, even chunk k+1, ... of this XCD's slab
-    const int par = qq & 1, pos = qq >> 1;
-    const int chunk = (L & 7) * ord.slab + (ord.paired == 2 ? (pos % ord.T) * ord.P + pos / ord.T : pos);
-    const int i = chunk * sites + lane;
-    s = par ? ord.half + i : i;
-    live = i < (par ? V - ord.half : ord.half);
-  } else {
-    const int chunk = (L & 7) * ord.slab + qq;
-    s = chunk * sites + lane;
-    live = s < V;
-  }
+  const bool live = ord_site(ord, sites, L & 7, qq, lane, V, &s);
 
   const uint32_t cs = sizeof(C);
   const uint32_t pl = (uint32_t)V * cs;     // one element plane
@@ -782,7 +770,9 @@ static int dslash_launch(susy_ctx *c, const typename CT<R>::t *src,
   }
   if (sign != 1 || p0 != nullptr || !c->doG) aux_out = nullptr;
 #if NCOL <= 4
-  const bool split = ds_split<R>(V), inl = split && c->doG && prep && !keep_prep && ds_split_inline(V);
+  const bool split = ds_split<R>(V);
+  // (an epilogue's launch has its pre-pass values from D)
+  const bool inl = split && c->doG && prep && !keep_prep && p0 == nullptr && ds_split_inline(V);
 #else
   const bool split = false, inl = false;
 #endif
@@ -826,8 +816,8 @@ static int dslash_launch(susy_ctx *c, const typename CT<R>::t *src,
 #define DS_GO(DAG, EPI)                                                                       \
   do {                                                                                        \
     if (inl)                                                                                  \
-      hipLaunchKernelGGL((k_dslash_split<R, DAG, EPI, NCOL == 2>), dim3(nb), dim3(threads),   \
-                         0, c->s, DS_ARGS);                                                   \
+      hipLaunchKernelGGL((k_dslash_split<R, DAG, EPI, NCOL == 2 && EPI == 0>), dim3(nb),      \
+                         dim3(threads), 0, c->s, DS_ARGS);                                    \
     else if (split)                                                                           \
       hipLaunchKernelGGL((k_dslash_split<R, DAG, EPI, false>), dim3(nb), dim3(threads), 0,    \
                          c->s, DS_ARGS);                                                      \
