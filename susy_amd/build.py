@@ -1,4 +1,4 @@
-"""Build libsusy_hip_U<N>.so (N = 2, 3, 4) for gfx950 with hipcc, in-tree.
+"""Build libsusy_hip_U<N>.so (N = 2, 3, 4, 5) for gfx950 with hipcc, in-tree.
 
 Every HIP source is compiled once per gauge group (NCOL is a compile-time
 constant, as in the reference's include/susy.h:16) and linked into

@@ -190,6 +190,11 @@ template <> struct DsSites<float> {
 //
 // A block covers ord.sites sites (at most DsSites::n, see ds_sites) of one
 // output component.  (Two threads sharing an output matrix: 10-15% slower.)
+// What bounds it on large lattices is the operand lines that L1 misses (U(4)
+// 16^3x32: 8.6e7 of 128 bytes a launch in FP64, 4.6e7 in FP32; 94 and 64 in
+// flight per CU at 480 and 370 cycles each).  The lines that the L2 misses are
+// not it alone: tiled orders of a layout of whole matrices halved them without
+// a matching gain in time.
 template <typename R, bool DAG, int EPI>
 __global__ void __launch_bounds__(DsSites<R>::n)
     __attribute__((amdgpu_waves_per_eu(DsSites<R>::waves)))
@@ -223,9 +228,9 @@ k_dslash(const typename CT<R>::t *__restrict__ src, typename CT<R>::t *__restric
 
   // The determinant sums' gathered scalars: 20 (site) or 4 (link) round trips
   // to memory one after the other were up to a third of a wave's time, so
-  // their loads go out together.  FP64 from U(4) on is bound by what the L2
-  // misses, and loses by it; so does FP32 at U(5), at every size (with the same
-  // three waves per SIMD).  us of a CG iteration, in turn | together: U(4) FP32
+  // their loads go out together.  FP64 from U(4) on has as many lines in flight
+  // as a CU keeps (94 at 16^3x32) and loses by it; so does FP32 at U(5), at every
+  // size (with the same three waves per SIMD).  us of a CG iteration, in turn | together: U(4) FP32
   // 8^3x16 107 | 99, 12^3x24 462 | 453, 16^4 738 | 730; U(3) FP64 8^3x16 89.3 |
   // 86.5, 16^4 712 | 706; but U(4) FP64 16^4 1337 | 1394, U(5) FP32 4^4 75 | 92,
   // 8^4 125 | 161, 8^3x16 176 | 211, 12^4 438 | 495, 16^4 1333 | 1438.
@@ -454,10 +459,13 @@ k_dslash(const typename CT<R>::t *__restrict__ src, typename CT<R>::t *__restric
 // plaquette, one half of Dplus or (w >= 2) one PtoP pair.  The determinant
 // terms' sums over neighbours are shared the same way.
 //
-// What bounds it is still latency: gathered loads, then LDS and two barriers.
+// What bounds it is still latency: gathered loads, then LDS and two barriers
+// (U(4) 6^3x10: 83% L2 hits, 27 lines in flight per CU in FP64 and 14 in FP32 at
+// 190-260 cycles each, waves waiting 44% of their time).
 // FP32 holds its partial matrices in two rounds of half the LDS and asks for
 // five waves per SIMD (U(4) D: four, what its registers allow without
-// scratch); FP64 asks for two, where fewer registers made it slower.
+// scratch); FP64 asks for two.  At U(4) its 87 KB of LDS leave a CU one block,
+// five waves, whatever its registers, so fewer registers gained nothing there.
 // D with its pre-pass, us, FP64 | FP32, k_dslash -> this kernel:
 //   U(4) 4^3x8 23.7 -> 10.2 | 19.0 -> 9.4, 6^3x10 27.9 -> 23.3 | 24.9 -> 15.6
 //   U(3) 4^3x8 15.5 -> 8.0 | 13.9 -> 7.4, 6^3x10 19.3 -> 15.2 | 18.2 -> 11.3

@@ -33,14 +33,16 @@ __device__ __forceinline__ double bcs(int t, int dt, int nt, double pbc) {
 // the Q-closed terms w and w + 4), their sums meet in LDS, and then each wave
 // makes a column of X.  One thread per link went through its 32 products and
 // the determinant's gathered scalars one after the other, which was all its
-// time on small lattices.  On large ones the lines that the XCDs' L2 miss
-// bound it: the blocks take the operator kernel's order of site chunks, so
-// the neighbourhoods shared by the directions and by the next chunks meet in
-// one XCD's L2.  A force with one pole (D, this and the update), us: U(4) 4^3x8
-// 166 -> 63, 8^3x16 238 -> 164, 16^4 1472 -> 1085; U(3) 4^4 106 -> 48, 16^4
-// 761 -> 603; U(2) 4^4 57 -> 36, 16^4 330 -> 233.  Five waves with SV on its
-// own leave three of eight wave slots empty (16^4: 1308 at U(4)), one wave a
-// link spills or takes 256 registers (2355).
+// time on small lattices.  On large ones it waits for gathered lines, half of
+// which the XCD's L2 misses (U(4) 16^4: 46% hits, 65 lines in flight per CU at
+// 465 cycles each, waves waiting 72% of their time): the blocks take the
+// operator kernel's order of site chunks, so the neighbourhoods shared by the
+// directions and by the next chunks meet in one XCD's L2.  A force with one
+// pole (D, this and the update), us: U(4) 4^3x8 166 -> 63, 8^3x16 238 -> 164,
+// 16^4 1472 -> 1085; U(3) 4^4 106 -> 48, 16^4 761 -> 603; U(2) 4^4 57 -> 36,
+// 16^4 330 -> 233.  Five waves with SV on its own leave three of eight wave
+// slots empty (16^4: 1308 at U(4)), one wave a link spills or takes 256
+// registers (2355).
 // auxS, auxP: Tr sol_site, Tr(U_a^-1 sol_a); Tr psol_site^dag,
 // Tr(U_a^-1 psol_a^dag).
 // (waves per SIMD: what the registers of two operands and X allow without

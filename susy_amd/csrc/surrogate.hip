@@ -15,7 +15,7 @@
 // U += eps mom): each loop contributes G (rest)^dag where U_a(x) appears and
 // conj(G) (rest) where U_a(x)^dag appears, G = (g_re + i g_im) / (2N) from
 // the feature gradients g = dS/dphi, "rest" being the loop's other factors
-// in cyclic order.  The link owning thread sums its 32 occurrences.
+// in cyclic order.  A link has 32 occurrences in loops; one block sums them.
 //
 // Force matching: loss = |F_theta - F*|^2 / |F*|^2.  With R = F_theta - F*,
 // d loss / dtheta = d/dtheta [ d/deps S_theta(phi + eps v) ] / |F*|^2, where
@@ -258,9 +258,10 @@ __device__ __forceinline__ double2 mtrace_mul(const Mat a, const Mat b) {
 }
 
 // ---------------------------------------------------------------------
-// features phi[k * V + y], one thread per site and loop (blockIdx.y < 30) or
-// link norm.  What bounds it on a small lattice is a loop's chain of loads
-// and products, on a large one what the XCDs' L2 miss; one thread per site
+// features phi[k * V + y], one thread per site and loop (part k < 30 of the
+// site's chunk) or link norm.  What bounds it is a loop's chain of gathered
+// loads and products: waves wait for two thirds of their time, on a small
+// lattice for want of waves, at 16^4 with 65% L2 hits.  One thread per site
 // walked all 30 loops (us: U(4) 4^3x8 306 -> 12, 16^4 508 -> 221, U(2) 16^4
 // 114 -> 36).
 #define SGF_B 64
@@ -476,10 +477,11 @@ k_sg_back0(const unsigned short *__restrict__ wbf, const float *__restrict__ gz1
 
 // F = dS/dUbar on link (x, a).  A block makes one link direction of 16
 // sites: its 32 groups of 16 lanes take one of the link's 32 occurrences each,
-// whose contributions meet in the wave and then in LDS.  Large lattices are
-// bound by the links' lines that the XCDs' L2 miss, small ones by one
-// occurrence's chain of loads and products; a thread that owned a link made
-// its 32 of them one after the other (us: U(4) 4^3x8 269 -> 15, 8^3x16 325 ->
+// whose contributions meet in the wave and then in LDS.  What bounds it is an
+// occurrence's chain of gathered loads and FP64 products, on large lattices
+// too: at U(4) 16^4 85% of the requests hit L2 and a CU has 19 lines in flight,
+// yet waves wait for 58% of their time.  A thread that owned a link made its
+// 32 occurrences one after the other (us: U(4) 4^3x8 269 -> 15, 8^3x16 325 ->
 // 166, 16^4 1542 -> 1368, U(2) 4^4 72 -> 6, 16^4 204 -> 206).  Four waves on 64
 // sites, eight occurrences each and no exchange between lanes, took 69, 213
 // and 1619 at the U(4) sizes.
