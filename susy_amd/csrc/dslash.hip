@@ -191,7 +191,7 @@ template <> struct DsSites<float> {
 // A block covers ord.sites sites (at most DsSites::n, see ds_sites) of one
 // output component.  (Two threads sharing an output matrix: 10-15% slower.)
 // What bounds it on large lattices is the operand lines that L1 misses (U(4)
-// 16^3x32: 8.6e7 of 128 bytes a launch in FP64, 4.6e7 in FP32; 94 and 64 in
+// 16^3x32: 8.6e7 of 128 bytes a launch in FP64, 4.6e7 in FP32; 96 and 65 in
 // flight per CU at 480 and 370 cycles each).  The lines that the L2 misses are
 // not it alone: tiled orders of a layout of whole matrices halved them without
 // a matching gain in time.
@@ -229,7 +229,7 @@ k_dslash(const typename CT<R>::t *__restrict__ src, typename CT<R>::t *__restric
   // The determinant sums' gathered scalars: 20 (site) or 4 (link) round trips
   // to memory one after the other were up to a third of a wave's time, so
   // their loads go out together.  FP64 from U(4) on has as many lines in flight
-  // as a CU keeps (94 at 16^3x32) and loses by it; so does FP32 at U(5), at every
+  // as a CU keeps (96 at 16^3x32) and loses by it; so does FP32 at U(5), at every
   // size (with the same three waves per SIMD).  us of a CG iteration, in turn | together: U(4) FP32
   // 8^3x16 107 | 99, 12^3x24 462 | 453, 16^4 738 | 730; U(3) FP64 8^3x16 89.3 |
   // 86.5, 16^4 712 | 706; but U(4) FP64 16^4 1337 | 1394, U(5) FP32 4^4 75 | 92,
@@ -460,7 +460,7 @@ k_dslash(const typename CT<R>::t *__restrict__ src, typename CT<R>::t *__restric
 // terms' sums over neighbours are shared the same way.
 //
 // What bounds it is still latency: gathered loads, then LDS and two barriers
-// (U(4) 6^3x10: 83% L2 hits, 27 lines in flight per CU in FP64 and 14 in FP32 at
+// (U(4) 6^3x10: 83% L2 hits, 38 lines in flight per CU in FP64 and 22 in FP32 at
 // 190-260 cycles each, waves waiting 44% of their time).
 // FP32 holds its partial matrices in two rounds of half the LDS and asks for
 // five waves per SIMD (U(4) D: four, what its registers allow without

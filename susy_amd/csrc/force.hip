@@ -34,7 +34,7 @@ __device__ __forceinline__ double bcs(int t, int dt, int nt, double pbc) {
 // makes a column of X.  One thread per link went through its 32 products and
 // the determinant's gathered scalars one after the other, which was all its
 // time on small lattices.  On large ones it waits for gathered lines, half of
-// which the XCD's L2 misses (U(4) 16^4: 46% hits, 65 lines in flight per CU at
+// which the XCD's L2 misses (U(4) 16^4: 46% hits, 66 lines in flight per CU at
 // 465 cycles each, waves waiting 72% of their time): the blocks take the
 // operator kernel's order of site chunks, so the neighbourhoods shared by the
 // directions and by the next chunks meet in one XCD's L2.  A force with one
