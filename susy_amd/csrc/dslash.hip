@@ -743,7 +743,9 @@ k_dslash_split(const typename CT<R>::t *__restrict__ src, typename CT<R>::t *__r
 //             16384: 64.7 | 64.1   32768: 111 | 110     65536: 191 | 192
 // U(2) FP32 gives the sizes between 3072 and 6144 back to k_dslash; 2% at 6144
 // and 8192 (and at 8192 in FP64) are left to this kernel, which is the faster
-// one at 6912 and from 9216 on, and alone at 6144 (10.7 us of 11.2).
+// one at 6912 and from 9216 on, and alone at 6144 (10.7 us of 11.2).  Between the
+// sizes measured on both sides of an upper limit up to 4% are left to k_dslash
+// (U(2) 12^3x24 FP64 198 | 192, FP32 136 | 131; U(4) 8^3x12 FP64 124 | 121).
 template <typename R>
 static bool ds_split(int V) {
   const bool dbl = sizeof(R) == sizeof(double);
